@@ -752,17 +752,21 @@ __device__ __forceinline__ int swzVd(int row) {  // 8 rows x 32 bytes per half-w
   return (row & 7) << 1;
 }
 
-template <int DP>
+template <int DP, int NW>
 struct SplitCfg {
-  static constexpr int NW = (DP == 256) ? 2 : 4;        // wavefronts per workgroup
-  static constexpr int STAGE = 2 * 32 * DP * 2;         // K block + V block, 32 rows each
-  static constexpr int RING = 2 * STAGE;                // per wavefront
-  static constexpr int LDS = NW * RING;
+  static constexpr int STAGE = 2 * 32 * DP * 2;  // K block + V block, 32 rows each
+  static constexpr int RING = 2 * STAGE;         // per wavefront
+  static constexpr int QB = 16 * DP * 2;         // per wavefront: its copy of the 16 q slots
+  static constexpr int LDS = NW * (RING + QB);
 };
 
-template <typename T, int DP, bool DROP = false>
-__global__ void __launch_bounds__(SplitCfg<DP>::NW * 64, 1) fa_splitkv_kernel(const KArgs a) {
-  constexpr int NW = SplitCfg<DP>::NW;
+// A wavefront keeps two 32-row blocks of K and V in flight; the rest of the kernel is arranged for latency, because a
+// slice may be one block per wavefront long: Q comes in by the same DMA as K (one wait for everything, where loads
+// under a condition were four round trips one after the other), both first blocks are requested before anything is
+// waited for, and the addresses of full blocks need only scalar arithmetic.
+template <typename T, int DP, int NW, bool DROP = false>
+__global__ void __launch_bounds__(NW * 64, 1) fa_splitkv_kernel(const KArgs a) {
+  using Cfg = SplitCfg<DP, NW>;
   constexpr int CPR = DP / 8;
   constexpr int ROWB = DP * 2;
   constexpr int BLK = 32 * ROWB;        // bytes of a 32-row K (or V) block
@@ -770,6 +774,9 @@ __global__ void __launch_bounds__(SplitCfg<DP>::NW * 64, 1) fa_splitkv_kernel(co
   constexpr int RPI = 64 / CPR;         // rows per DMA instruction
   constexpr int KS = DP / 32;           // k-steps of the 16x16x32 MFMA over head dim
   constexpr int MB = DP / 16;           // 16-row blocks of O^T
+  // consecutive DMA instructions are RPI rows apart; after NVK (NVV) of them the row's swizzle repeats
+  constexpr int NVK = 16 / RPI;
+  constexpr int NVV = DP == 64 ? 1 : 8 / RPI;
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
 
   const int tid = threadIdx.x;
@@ -794,14 +801,16 @@ __global__ void __launch_bounds__(SplitCfg<DP>::NW * 64, 1) fa_splitkv_kernel(co
     lb = (int64_t)q0 * a.lse_ss;
   }
   if (a.seqused_k) Lk = min(Lk, max(a.seqused_k[b], 0));
+  if (Lq <= 0) return;
   const int D = a.head_dim;
   const int group = a.group;
   const int h0 = hk * group;
   // q slot L of the MFMA's N dimension <-> (query row L / group, head h0 + L % group); slots >= nslots are zero
   // (packed: a sequence longer than the seqlen_q the caller gave is cut to its first seqlen_q rows — the 16 MFMA
   // columns and the workspace are sized by it; the causal alignment below keeps the true length)
-  const int nslots = group * max(min(Lq, a.seqlen_q), 0);
-  const int slot_r = L / group, slot_g = L % group;
+  const int nslots = group * min(Lq, a.seqlen_q);
+  const unsigned inv_group = (65536u + group - 1) / (unsigned)group;  // slot / group = slot * inv_group >> 16 (slot < 16)
+  const int slot_r = (int)((unsigned)L * inv_group >> 16), slot_g = L - slot_r * group;
   // keys this lane's slot may see: bottom-right causal lets row r see keys <= Lk - Lq + r
   const int slot_lim = a.is_causal ? min(Lk - 1, Lk - Lq + slot_r) : Lk - 1;
   const int mask_from = a.is_causal ? Lk - (Lq - 1) : Lk;  // first key that some slot does not see
@@ -825,71 +834,93 @@ __global__ void __launch_bounds__(SplitCfg<DP>::NW * 64, 1) fa_splitkv_kernel(co
   const int per = (nblk + a.n_splits - 1) / a.n_splits;
   const int blk_begin = split * per;
   const int blk_end = min(nblk, blk_begin + per);
-  const int last_k = Lk - 1;
+  const int blk0 = blk_begin + wave;
+  const int n_my = max(0, (blk_end - blk0 + NW - 1) / NW);
 
   const unsigned char* kp = a.k + kb + (int64_t)k0 * a.k_ss + (int64_t)hk * a.k_sh;
   const unsigned char* vp = a.v + vb + (int64_t)k0 * a.v_ss + (int64_t)hk * a.v_sh;
   const unsigned k_ss = (unsigned)a.k_ss, v_ss = (unsigned)a.v_ss;
+  const unsigned lds0 = (unsigned)(uintptr_t)(LDS_AS unsigned char*)smem;
+  const unsigned ring = lds0 + wave * Cfg::RING, qlds = lds0 + NW * Cfg::RING + wave * Cfg::QB;
 
-  unsigned char* ring = smem + wave * SplitCfg<DP>::RING;
+  // ---- DMA bookkeeping: instruction i of a block fills LDS rows RPI i + dma_r; chunk un-swizzled on the global side ----
   const int dma_r = lane / CPR, dma_pc = lane % CPR;
+  auto chunk_k = [&](int i) {
+    const int lc = dma_pc ^ swzKd<DP>(dma_r + i * RPI);
+    return lc * 8 < D ? lc : 0;
+  };
+  auto chunk_v = [&](int i) {
+    const int lc = dma_pc ^ swzVd<DP>(dma_r + i * RPI);
+    return lc * 8 < D ? lc : 0;
+  };
+  unsigned koff[NVK], voff[NVV];
+#pragma unroll
+  for (int i = 0; i < NVK; ++i) koff[i] = dma_r * k_ss + chunk_k(i) * 16;
+#pragma unroll
+  for (int i = 0; i < NVV; ++i) voff[i] = dma_r * v_ss + chunk_v(i) * 16;
 
   // Paged cache: a 32-row block lies inside one page (page_size is a multiple of 32), so the page is one scalar
-  // table entry per block; `page` is that entry (fetched an iteration ahead of its use) and the rows count from the
-  // page's first row.  Without a table `page` is 0 and the rows count from the sequence's first key.
+  // table entry per block, requested a block ahead of its use; (pg_idx, pg_in) walks (entry, block in the page) without
+  // a division.
   const int32_t* tbl = a.block_table ? a.block_table + (int64_t)b * a.bt_stride : nullptr;
-  const int psz = a.page_size;
-  auto page_of = [&](int blk_) -> int { return tbl ? tbl[min(blk_ * 32, last_k) / psz] : 0; };
+  const int bpp = tbl ? a.page_size >> 5 : 1;  // blocks per page
+  int pg_idx = 0, pg_in = 0;
+  if (tbl) {
+    pg_idx = blk0 / bpp;
+    pg_in = blk0 - pg_idx * bpp;
+    kp = a.k + (int64_t)hk * a.k_sh;
+    vp = a.v + (int64_t)hk * a.v_sh;
+  }
+  auto lookup = [&](bool exists) { return tbl && exists ? __builtin_amdgcn_readfirstlane(tbl[pg_idx]) : 0; };
+  // fetch block blk (this wavefront's next one) into `stage`; page: its table entry
   auto issue_block = [&](int blk, int stage, int page) {
-    unsigned char* kdst = ring + stage * SplitCfg<DP>::STAGE;
-    unsigned char* vdst = kdst + BLK;
-    const unsigned char* kpg = kp;
-    const unsigned char* vpg = vp;
-    int row0 = 0;  // first key row of what kpg / vpg point at
+    const unsigned dst = ring + stage * Cfg::STAGE;
+    const unsigned row0 = tbl ? (unsigned)pg_in * 32u : (unsigned)blk * 32u;
+    const unsigned char* kt = kp + (tbl ? (int64_t)page * a.k_sb : 0) + (uint64_t)row0 * k_ss;
+    const unsigned char* vt = vp + (tbl ? (int64_t)page * a.v_sb : 0) + (uint64_t)row0 * v_ss;
     if (tbl) {
-      kpg = a.k + (int64_t)page * a.k_sb + (int64_t)hk * a.k_sh;
-      vpg = a.v + (int64_t)page * a.v_sb + (int64_t)hk * a.v_sh;
-      row0 = min(blk * 32, last_k) / psz * psz;
+      pg_in += NW;
+      while (pg_in >= bpp) {
+        pg_in -= bpp;
+        ++pg_idx;
+      }
     }
+    const int rmax = Lk - 1 - blk * 32;
+    if (rmax >= 31) {
 #pragma unroll
-    for (int i = 0; i < NI; ++i) {
-      const int r = dma_r + i * RPI;
-      int lc = dma_pc ^ swzKd<DP>(r);
-      if (lc * 8 >= D) lc = 0;
-      const int gr = min(blk * 32 + r, last_k) - row0;
-      dma16(kpg + (uint64_t)(unsigned)gr * k_ss + lc * 16, kdst + i * 1024);
-    }
+      for (int i = 0; i < NI; ++i) dma16s(kt + (uint64_t)(unsigned)(i * RPI) * k_ss, koff[i % NVK], dst + i * 1024);
 #pragma unroll
-    for (int i = 0; i < NI; ++i) {
-      const int r = dma_r + i * RPI;
-      int lc = dma_pc ^ swzVd<DP>(r);
-      if (lc * 8 >= D) lc = 0;
-      const int gr = min(blk * 32 + r, last_k) - row0;
-      dma16(vpg + (uint64_t)(unsigned)gr * v_ss + lc * 16, vdst + i * 1024);
+      for (int i = 0; i < NI; ++i) dma16s(vt + (uint64_t)(unsigned)(i * RPI) * v_ss, voff[i % NVV], dst + BLK + i * 1024);
+    } else {  // the last block of the sequence: rows clamped to its last one
+#pragma unroll
+      for (int i = 0; i < NI; ++i) dma16s(kt, (unsigned)min(dma_r + i * RPI, rmax) * k_ss + chunk_k(i) * 16, dst + i * 1024);
+#pragma unroll
+      for (int i = 0; i < NI; ++i) dma16s(vt, (unsigned)min(dma_r + i * RPI, rmax) * v_ss + chunk_v(i) * 16, dst + BLK + i * 1024);
     }
   };
 
-  int blk = blk_begin + wave;
-  const bool any = blk < blk_end && Lq > 0;
-  if (any) issue_block(blk, 0, page_of(blk));
-  int page_next = (any && blk + NW < blk_end) ? page_of(blk + NW) : 0;  // the table entry of the next block to fetch
-
   // Q^T as B operand of 16x16x32: lane (q slot = L, G) holds Q[row][head][32 ks + 8 G .. +8] of its slot
   s16x8 qf[KS];
-  {
-    const unsigned flip = a.neg_scale ? 0x80008000u : 0u;
-    const unsigned char* qrow = a.q + qb + (int64_t)(q0 + slot_r) * a.q_ss + (int64_t)(h0 + slot_g) * a.q_sh;
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-      const int ch = 4 * ks + G;
-      u32x4 x = {0, 0, 0, 0};
-      if (L < nslots && ch * 8 < D) {
-        x = *(const u32x4*)(qrow + ch * 16);
-        x ^= flip;
+  for (int ks = 0; ks < KS; ++ks) qf[ks] = s16x8{0, 0, 0, 0, 0, 0, 0, 0};
+  if (n_my > 0) {
+    int page = lookup(true);
+    {
+      const unsigned char* qh = a.q + qb + (int64_t)q0 * a.q_ss + (int64_t)h0 * a.q_sh;
+#pragma unroll
+      for (int i = 0; i < 16 / RPI; ++i) {
+        const unsigned slot = (unsigned)min(dma_r + i * RPI, nslots - 1);
+        const unsigned r = slot * inv_group >> 16;
+        dma16v(qh + (int64_t)r * a.q_ss + (int64_t)(slot - r * group) * a.q_sh + chunk_k(i) * 16, qlds + i * 1024);
       }
-      qf[ks] = __builtin_bit_cast(s16x8, x);
+    }
+    issue_block(blk0, 0, page);
+    if (n_my > 1) {
+      page = lookup(true);
+      issue_block(blk0 + NW, 1, page);
     }
   }
+  int page_next = lookup(n_my > 2);
 
   f32x4 o[MB];
 #pragma unroll
@@ -903,19 +934,29 @@ __global__ void __launch_bounds__(SplitCfg<DP>::NW * 64, 1) fa_splitkv_kernel(co
   const int v_lane_off = vrow * ROWB + (L & 1) * 8;
   const int v_lc0 = (L & 3) >> 1;
 
-  int stage = 0;
-  for (; blk < blk_end && Lq > 0; blk += NW) {
-    const int nxt = blk + NW;
-    if (nxt < blk_end) {
-      issue_block(nxt, stage ^ 1, page_next);
-      page_next = (nxt + NW < blk_end) ? page_of(nxt + NW) : 0;
+  for (int it = 0; it < n_my; ++it) {
+    const int blk = blk0 + it * NW, stage = it & 1;
+    // this block has landed (loads retire in order); the next one may still be in flight
+    if (it + 1 < n_my) {
       if constexpr (NI == 4) WAIT_VMCNT(8);
       else if constexpr (NI == 8) WAIT_VMCNT(16);
       else WAIT_VMCNT(32);
     } else {
       WAIT_VMCNT(0);
     }
-    const unsigned char* kt = ring + stage * SplitCfg<DP>::STAGE;
+    if (it == 0) {
+      const unsigned flip = a.neg_scale ? 0x80008000u : 0u;
+      const unsigned char* qs = smem + NW * Cfg::RING + wave * Cfg::QB;
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+        const int ch = 4 * ks + G;
+        u32x4 x = *(const u32x4*)(qs + L * ROWB + (ch ^ ksw) * 16);
+        x ^= flip;
+        if (L >= nslots || ch * 8 >= D) x = u32x4{0, 0, 0, 0};
+        qf[ks] = __builtin_bit_cast(s16x8, x);
+      }
+    }
+    const unsigned char* kt = smem + wave * Cfg::RING + stage * Cfg::STAGE;
     const unsigned char* vt = kt + BLK;
 
     // S^T (kv x q slot): two 16-row tiles
@@ -991,58 +1032,54 @@ __global__ void __launch_bounds__(SplitCfg<DP>::NW * 64, 1) fa_splitkv_kernel(co
       const s16x8 av = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
       o[mb] = Mma<T>::m16(av, pb, o[mb]);
     }
-    stage ^= 1;
+    if (it + 2 < n_my) {
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // every read of this stage is done
+      issue_block(blk + 2 * NW, stage, page_next);
+      page_next = lookup(it + 3 < n_my);
+    }
   }
 
   // ---- merge the NW wavefronts' partials through LDS ----
   l_run += __shfl_xor(l_run, 16);
   l_run = pair_sum32(l_run);
   __syncthreads();  // all rings are idle (every wavefront waited for its last DMA before its last block)
-  float* so = (float*)smem;                       // [NW][16][DP]
-  float* sml = (float*)(smem + NW * 16 * DP * 4); // [NW][16][2]
+  constexpr int OS = DP + 4;                      // row stride in floats
+  float* so = (float*)smem;                       // [NW][16][OS]
+  float* sml = (float*)(smem + NW * 16 * OS * 4); // [NW][16][2]
+  if (L < nslots) {
 #pragma unroll
-  for (int mb = 0; mb < MB; ++mb)
-#pragma unroll
-    for (int v = 0; v < 4; ++v) so[(wave * 16 + L) * DP + 16 * mb + 4 * G + v] = o[mb][v];
-  if (G == 0) {
-    sml[(wave * 16 + L) * 2 + 0] = (m_run == -INFINITY) ? -INFINITY : m_run * c;
-    sml[(wave * 16 + L) * 2 + 1] = l_run;
+    for (int mb = 0; mb < MB; ++mb) *(f32x4*)(so + (wave * 16 + L) * OS + 16 * mb + 4 * G) = o[mb];
+    if (G == 0) {
+      sml[(wave * 16 + L) * 2 + 0] = (m_run == -INFINITY) ? -INFINITY : m_run * c;
+      sml[(wave * 16 + L) * 2 + 1] = l_run;
+    }
   }
   __syncthreads();
-  if (Lq <= 0) return;
-  // thread -> (q slot, 16 d-values)
-  constexpr int TPQ = DP / 16;  // threads per q slot
+  // thread -> (q slot, 4 d-values)
+  constexpr int TPQ = DP / 4;
   for (int item = tid; item < nslots * TPQ; item += NW * 64) {
-    const int qs = item / TPQ, d0 = (item % TPQ) * 16;
-    float M = -INFINITY;
+    const int qs = item / TPQ, d0 = (item % TPQ) * 4;
+    float mw[NW], M = -INFINITY;
 #pragma unroll
-    for (int w = 0; w < NW; ++w) M = fmaxf(M, sml[(w * 16 + qs) * 2]);
-    float acc[16];
-#pragma unroll
-    for (int i = 0; i < 16; ++i) acc[i] = 0.f;
+    for (int w = 0; w < NW; ++w) {
+      mw[w] = sml[(w * 16 + qs) * 2];
+      M = fmaxf(M, mw[w]);
+    }
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
     float lsum = 0.f;
 #pragma unroll
     for (int w = 0; w < NW; ++w) {
-      const float mw = sml[(w * 16 + qs) * 2];
-      const float sc = (mw == -INFINITY) ? 0.f : fast_exp2(mw - M);
+      const float sc = (mw[w] == -INFINITY) ? 0.f : fast_exp2(mw[w] - M);
       lsum += sml[(w * 16 + qs) * 2 + 1] * sc;
-#pragma unroll
-      for (int i = 0; i < 16; ++i) acc[i] += so[(w * 16 + qs) * DP + d0 + i] * sc;
+      acc += *(const f32x4*)(so + (w * 16 + qs) * OS + d0) * sc;
     }
-    const int qr = qs / group;  // query row of this slot (0 in packed mode)
-    const int h = h0 + qs % group;
+    const int qr = (int)((unsigned)qs * inv_group >> 16);  // query row of this slot (0 in packed mode)
+    const int h = h0 + qs - qr * group;
     if (a.n_splits == 1) {
       const float inv = (lsum > 0.f) ? (DROP ? a.drop_rp : 1.f) / lsum : 0.f;
       if (d0 < D) {
         unsigned char* orow = a.out + ob + (int64_t)(q0 + qr) * a.o_ss + (int64_t)h * a.o_sh + d0 * 2;
-        u32x4 w0, w1;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          w0[i] = Mma<T>::pack2(acc[2 * i] * inv, acc[2 * i + 1] * inv);
-          w1[i] = Mma<T>::pack2(acc[8 + 2 * i] * inv, acc[8 + 2 * i + 1] * inv);
-        }
-        *(u32x4*)orow = w0;
-        if (d0 + 8 < D) *(u32x4*)(orow + 16) = w1;
+        *(u32x2*)orow = u32x2{Mma<T>::pack2(acc[0] * inv, acc[1] * inv), Mma<T>::pack2(acc[2] * inv, acc[3] * inv)};
       }
       if (d0 == 0)
         a.lse[lb + (int64_t)h * a.lse_sh + (int64_t)qr * a.lse_ss] = (lsum > 0.f) ? (M + __builtin_log2f(lsum)) * kLn2 : INFINITY;
@@ -1050,27 +1087,23 @@ __global__ void __launch_bounds__(SplitCfg<DP>::NW * 64, 1) fa_splitkv_kernel(co
       // one slot per (sequence, head, query row, slice): what fa_merge_rows_kernel reads (packed: seqlen_q is the
       // longest sequence, shorter ones leave their last slots unused)
       const int64_t slot = (((int64_t)b * a.heads_q + h) * a.seqlen_q + qr) * a.n_splits + split;
-      if (d0 < D) {
-        float* dst = a.ws_o + slot * D + d0;
-#pragma unroll
-        for (int i = 0; i < 16; ++i)
-          if (d0 + i < D) dst[i] = acc[i];
-      }
-      if (d0 == 0) {
-        a.ws_ml[slot * 2 + 0] = M;
-        a.ws_ml[slot * 2 + 1] = lsum;
-      }
+      if (d0 < D) *(f32x4*)(a.ws_o + slot * D + d0) = acc;
+      if (d0 == 0) *(f32x2*)(a.ws_ml + slot * 2) = f32x2{M, lsum};
     }
   }
 }
 
-// Merge the per-slice partials of either kernel: one wavefront per (sequence, query head, query row), four rows per
-// workgroup; lane -> head_dim elements lane, lane+64, ...  Packed mode: seqlen_q is the longest sequence; rows beyond
-// a sequence's own length have no partials and are skipped.
-template <typename T>
+// Merge the per-slice partials of either kernel.  WPR wavefronts work on one row (sequence, query head, query row):
+// 4 where the rows are too few to fill the chip with one each (decode), otherwise 1.  A lane takes 4 head_dim elements
+// of every SPW-th slice, so that one load instruction covers 1 KiB and the loads of all slices are in flight together:
+// what is left is about one memory latency.  Packed mode: seqlen_q is the longest sequence; rows beyond a sequence's own
+// length have no partials and are skipped.
+template <typename T, int WPR>
 __global__ void __launch_bounds__(256) fa_merge_rows_kernel(const KArgs a) {
   const int lane = threadIdx.x & 63;
-  const int64_t r = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);  // (b * heads_q + h) * seqlen_q + row
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wr = WPR == 4 ? wave : 0;  // this wavefront among those of its row
+  const int64_t r = WPR == 4 ? (int64_t)blockIdx.x : (int64_t)blockIdx.x * 4 + wave;  // (b * heads_q + h) * seqlen_q + row
   const int64_t rows = (int64_t)a.batch * a.heads_q * a.seqlen_q;
   if (r >= rows) return;
   const int row = (int)(r % a.seqlen_q);
@@ -1087,39 +1120,59 @@ __global__ void __launch_bounds__(256) fa_merge_rows_kernel(const KArgs a) {
   }
   const float* ml = a.ws_ml + r * ns * 2;
   const float* po = a.ws_o + r * ns * D;
-  // lane s holds slice s's (m, l) (at most 64 slices); the maximum, the scale factors and the sum of l are formed
-  // across the wavefront, then the slices' rows are accumulated with independent loads
-  float ms = -INFINITY, ls = 0.f;
-  if (lane < ns) {
-    const f32x2 v = *(const f32x2*)(ml + 2 * lane);
-    ms = v[0];
-    ls = v[1];
-  }
-  float M = ms;
+  const int lps = D <= 64 ? 16 : (D <= 128 ? 32 : 64);  // lanes per slice
+  const int spw = 64 / lps;                             // slices per load instruction
+  const int sub = lane / lps, d0 = (lane % lps) * 4;
+  // lane s holds slice s's (m, l) (at most 64 slices)
+  f32x2 v = {-INFINITY, 0.f};
+  if (lane < ns) v = *(const f32x2*)(ml + 2 * lane);
+  constexpr int U = 4;
+  const int s_step = WPR * spw;
+  const int d_ld = min(d0, D - 4);  // lanes beyond head_dim read a valid piece and are dropped at the end
+  f32x4 x[U];
+  auto load = [&](int s0) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int s = s0 + u * s_step;
+      x[u] = *(const f32x4*)(po + (int64_t)min(s, ns - 1) * D + d_ld);
+    }
+  };
+  int s0 = wr * spw + sub;
+  load(s0);
+  float M = v[0];
 #pragma unroll
   for (int o = 32; o >= 1; o >>= 1) M = fmaxf(M, __shfl_xor(M, o));
-  const float scl = (ms == -INFINITY) ? 0.f : fast_exp2(ms - M);  // 0: a slice without a visible key for this row
-  float lsum = ls * scl;
+  const float scl = (v[0] == -INFINITY) ? 0.f : fast_exp2(v[0] - M);  // 0: a slice without a visible key for this row
+  float lsum = v[1] * scl;
 #pragma unroll
   for (int o = 32; o >= 1; o >>= 1) lsum += __shfl_xor(lsum, o);
-  float acc[4] = {0.f, 0.f, 0.f, 0.f};  // head_dim <= 256
-#pragma unroll 4
-  for (int s = 0; s < ns; ++s) {
-    const float sc = __shfl(scl, s);
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  for (;;) {
+    // a slice that saw no key leaves zeros (the tile kernel) or finite partial sums; its factor is 0 either way
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int d = lane + 64 * i;
-      // a slice that saw no key leaves zeros (the tile kernel) or finite partial sums; its factor is 0 either way
-      if (d < D) acc[i] += po[(int64_t)s * D + d] * sc;
+    for (int u = 0; u < U; ++u) {
+      const int s = s0 + u * s_step;
+      const float f = __shfl(scl, min(s, 63));
+      acc += x[u] * (s < ns ? f : 0.f);
     }
+    s0 += U * s_step;
+    if (s0 - sub - wr * spw >= ns) break;  // (uniform over the wavefronts of the row)
+    load(s0);
+  }
+  for (int o = lps; o < 64; o <<= 1)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) acc[i] += __shfl_xor(acc[i], o);
+  if constexpr (WPR == 4) {
+    __shared__ f32x4 part[4][64];
+    part[wave][lane] = acc;
+    __syncthreads();
+    if (wave != 0) return;
+    acc = part[0][lane] + part[1][lane] + part[2][lane] + part[3][lane];
   }
   const float inv = (lsum > 0.f) ? a.drop_rp / lsum : 0.f;  // 1 / keep: the split-KV kernel's partials under dropout
-  T* orow = (T*)(a.out + orow_off + (int64_t)h * a.o_sh);
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int d = lane + 64 * i;
-    if (d < D) orow[d] = (T)(acc[i] * inv);
-  }
+  if (sub == 0 && d0 < D)
+    *(u32x2*)(a.out + orow_off + (int64_t)h * a.o_sh + d0 * 2) =
+        u32x2{Mma<T>::pack2(acc[0] * inv, acc[1] * inv), Mma<T>::pack2(acc[2] * inv, acc[3] * inv)};
   if (lane == 0)
     a.lse[lse_off + (int64_t)h * a.lse_sh] = (lsum > 0.f) ? (M + __builtin_log2f(lsum)) * kLn2 : INFINITY;
 }
@@ -1178,6 +1231,15 @@ KArgs make_args(const fa_fwd_params* p, int kern, int ns, void* ws) {
   return a;
 }
 
+template <typename T>
+int launch_merge(const KArgs& a, hipStream_t st) {
+  const int64_t rows = (int64_t)a.batch * a.heads_q * a.seqlen_q;
+  // four wavefronts a row until one each would give every CU two workgroups
+  if (rows < 2048) hipLaunchKernelGGL((fa_merge_rows_kernel<T, 4>), dim3((unsigned)rows), dim3(256), 0, st, a);
+  else hipLaunchKernelGGL((fa_merge_rows_kernel<T, 1>), dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, st, a);
+  return hipGetLastError() == hipSuccess ? FA_OK : FA_ERR_LAUNCH;
+}
+
 template <typename T, int DP, int MINB, int BIAS, bool DROP = false, bool DMASK = false, bool PAGED = false>
 int launch_tile(KArgs a, hipStream_t st) {
   constexpr int lds = 4 * 64 * DP * 2 + (BIAS == 2 ? 4 * 4096 : 0);
@@ -1207,43 +1269,38 @@ int launch_tile(KArgs a, hipStream_t st) {
   if (grid > 0x7fffffffLL) return FA_ERR_UNSUPPORTED;
   hipLaunchKernelGGL(kfn, dim3((unsigned)grid), dim3(256), lds, st, a);
   if (hipGetLastError() != hipSuccess) return FA_ERR_LAUNCH;
-  if (a.n_splits > 1) {
-    const int64_t rows = (int64_t)a.batch * a.heads_q * a.seqlen_q;
-    hipLaunchKernelGGL(fa_merge_rows_kernel<T>, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, st, a);
-    if (hipGetLastError() != hipSuccess) return FA_ERR_LAUNCH;
-  }
-  return FA_OK;
+  return a.n_splits > 1 ? launch_merge<T>(a, st) : FA_OK;
 }
 
-template <typename T, int DP, bool DROP>
+template <typename T, int DP, int NW, bool DROP>
 int launch_splitkv(const KArgs& a, hipStream_t st) {
-  constexpr int lds = SplitCfg<DP>::LDS;
-  constexpr auto kfn = fa_splitkv_kernel<T, DP, DROP>;
+  constexpr int lds = SplitCfg<DP, NW>::LDS;
+  constexpr auto kfn = fa_splitkv_kernel<T, DP, NW, DROP>;
   if (!ensure_dynamic_lds<kfn>(lds)) return FA_ERR_LAUNCH;
   const int64_t grid = (int64_t)a.batch * a.heads_k * a.n_splits;
   if (grid > 0x7fffffffLL) return FA_ERR_UNSUPPORTED;
-  hipLaunchKernelGGL(kfn, dim3((unsigned)grid), dim3(SplitCfg<DP>::NW * 64), lds, st, a);
+  hipLaunchKernelGGL(kfn, dim3((unsigned)grid), dim3(NW * 64), lds, st, a);
   if (hipGetLastError() != hipSuccess) return FA_ERR_LAUNCH;
-  if (a.n_splits > 1) {
-    const int64_t rows = (int64_t)a.batch * a.heads_q * a.seqlen_q;
-    hipLaunchKernelGGL(fa_merge_rows_kernel<T>, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, st, a);
-    if (hipGetLastError() != hipSuccess) return FA_ERR_LAUNCH;
-  }
-  return FA_OK;
+  return a.n_splits > 1 ? launch_merge<T>(a, st) : FA_OK;
+}
+
+// Sequences of one length: four wavefronts and most of a CU's LDS per workgroup, whose slices are equal and in step
+// (6.0 TB/s at B = 64, 8192 keys; two wavefronts: 5.6).  Ragged lengths: half the size, so that two workgroups share a CU
+// and one's start and merge are covered by the other's loads (32 sequences of 1024 ... 4096 keys: 73 against 80 us).
+template <typename T, bool DROP>
+int dispatch_splitkv(const KArgs& a, int dp, hipStream_t st) {
+  const bool ragged = a.seqused_k || a.cu_q;
+  if (dp == 64) return ragged ? launch_splitkv<T, 64, 2, DROP>(a, st) : launch_splitkv<T, 64, 4, DROP>(a, st);
+  if (dp == 128) return ragged ? launch_splitkv<T, 128, 2, DROP>(a, st) : launch_splitkv<T, 128, 4, DROP>(a, st);
+  return launch_splitkv<T, 256, 2, DROP>(a, st);
 }
 
 template <typename T>
 int dispatch(const KArgs& a, int kern, hipStream_t st) {
   const int dp = padded_dim(a.head_dim);
   if (kern == FA_KERNEL_SPLITKV) {
-    if (a.drop_thr < 255u) {  // dropout_p > 0
-      if (dp == 64) return launch_splitkv<T, 64, true>(a, st);
-      if (dp == 128) return launch_splitkv<T, 128, true>(a, st);
-      return launch_splitkv<T, 256, true>(a, st);
-    }
-    if (dp == 64) return launch_splitkv<T, 64, false>(a, st);
-    if (dp == 128) return launch_splitkv<T, 128, false>(a, st);
-    return launch_splitkv<T, 256, false>(a, st);
+    if (a.drop_thr < 255u) return dispatch_splitkv<T, true>(a, dp, st);  // dropout_p > 0
+    return dispatch_splitkv<T, false>(a, dp, st);
   }
   if (a.drop_thr < 255u && a.dmask) {  // dropout_p > 0 and the keep-mask is wanted (tests)
     if (a.bias) {
