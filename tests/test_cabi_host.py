@@ -225,6 +225,20 @@ def test_bwd_validate_accepts_good_params_and_sizes_delta_scratch():
     assert L.fa_bwd_validate(ctypes.byref(full)) == capi.FA_OK
 
 
+@pytest.mark.parametrize("Hq,Hk,S,D,slices", [
+    (28, 4, 4096, 128, 16),   # 448 steps, 112 a CU: slices of 28
+    (14, 2, 130, 128, 2),     # 21 steps: slices of 11
+    (16, 16, 2048, 128, 1),   # 32 steps, 16 a CU
+    (32, 32, 4096, 128, 1),
+    (16, 4, 2048, 64, 8),     # 128 steps, slices of 16
+])
+def test_bwd_workspace_holds_the_slices_partial_sums(Hq, Hk, S, D, slices):
+    p = _good_bwd(batch=1, heads_q=Hq, heads_k=Hk, seqlen_q=S, seqlen_k=S, head_dim=D)
+    planes = 2 * (S * Hq * 4)
+    parts = 0 if slices == 1 else Hk * ((S + 127) // 128) * slices * 2 * (128 * D * 4)
+    assert capi.lib().fa_bwd_workspace_bytes(ctypes.byref(p)) == planes + parts
+
+
 @pytest.mark.parametrize("over,rc", [
     (dict(dout=None), capi.FA_ERR_BAD_ARG),
     (dict(dk=None), capi.FA_ERR_BAD_ARG),

@@ -70,3 +70,70 @@ def test_decode_slices_around_the_blocks_of_a_wavefront(D, used):
         want = torch.exp(s - want_l[..., None]) @ v[:, :, :n].float().repeat_interleave(3, 1)
         assert (out.float() - want).abs().max().item() <= OUT_TOL[BF]
         assert (lse - want_l).abs().max().item() <= LSE_TOL
+
+
+def _grad_reference(q, k, v, do, causal, bias=None):
+    """Gradients of one dense call in float64 on the CPU."""
+    q, k, v, do = (t.double().cpu() for t in (q, k, v, do))
+    g, D, Sq, Sk = q.shape[1] // k.shape[1], q.shape[3], q.shape[2], k.shape[2]
+    kr, vr = k.repeat_interleave(g, 1), v.repeat_interleave(g, 1)
+    s = q @ kr.transpose(2, 3) / math.sqrt(D)
+    if bias is not None:
+        s = s + bias.double().cpu()
+    if causal:
+        s.masked_fill_(~(torch.arange(Sk)[None, :] <= torch.arange(Sq)[:, None] + Sk - Sq), float("-inf"))
+    p = torch.nan_to_num(torch.softmax(s, -1))
+    dp = do @ vr.transpose(2, 3)
+    ds = p * (dp - (p * dp).sum(-1, keepdim=True)) / math.sqrt(D)
+    B, Hk = k.shape[:2]
+    fold = lambda t: t.reshape(B, Hk, g, Sk, D).sum(2)
+    return ds @ kr, fold(ds.transpose(2, 3) @ q), fold(p.transpose(2, 3) @ do)
+
+
+def _check_grads(got, want, dtype):
+    eps = 2.0 ** -8 if dtype == BF else 2.0 ** -11
+    for name, x, w in zip(("dq", "dk", "dv"), got, want):
+        x = x.double().cpu()
+        assert torch.isfinite(x).all(), name
+        # two units in the last place at the gradient's largest value, as for every backward test
+        assert (x - w).abs().max().item() <= 2 * eps * max(w.abs().max().item(), 0.25), name
+
+
+@pytest.mark.parametrize("D", [64, 72, 128, 256])
+@pytest.mark.parametrize("B,Hq,Hk,Sq,Sk,causal", [
+    (1, 14, 2, 130, 130, True),     # 21 and 7 steps: two slices, then one
+    (1, 14, 2, 300, 500, True),     # more keys than queries, 8 (sequence, kv head, block) units
+    (2, 21, 3, 500, 129, True),     # rows that see no key; a last block of one key
+    (1, 12, 1, 1024, 256, False),   # equal slices
+    (1, 2, 2, 1900, 64, False),     # one head's query tiles cut into slices
+])
+def test_sliced_key_blocks(D, B, Hq, Hk, Sq, Sk, causal):
+    for dt in (BF, HF):
+        q, k, v, do = (_randn(s, 20 + i, dt) for i, s in enumerate(
+            [(B, Hq, Sq, D), (B, Hk, Sk, D), (B, Hk, Sk, D), (B, Hq, Sq, D)]))
+        out, lse = capi.fa_forward_dense(q, k, v, is_causal=causal)
+        _check_grads(capi.fa_backward_dense(do, q, k, v, out, lse, is_causal=causal), _grad_reference(q, k, v, do, causal), dt)
+
+
+@pytest.mark.parametrize("D", [64, 128])
+def test_sliced_key_blocks_with_a_bias(D):
+    q, k, v, do = _randn((1, 14, 260, D), 30, BF), _randn((1, 2, 200, D), 31, BF), _randn((1, 2, 200, D), 32, BF), _randn((1, 14, 260, D), 33, BF)
+    bias = _randn((1, 1, 260, 200), 34, BF)
+    out, lse = capi.fa_forward_dense(q, k, v, bias=bias)
+    _check_grads(capi.fa_backward_dense(do, q, k, v, out, lse, bias=bias)[:3], _grad_reference(q, k, v, do, False, bias), BF)
+
+
+@pytest.mark.parametrize("Hq,Hk,D", [(14, 2, 64), (14, 2, 128), (8, 1, 96)])
+def test_sliced_key_blocks_packed(Hq, Hk, D):
+    lens = [1, 300, 64, 0, 129, 610]
+    cu = [0]
+    for n in lens:
+        cu.append(cu[-1] + n)
+    q, k, v, do = _randn((cu[-1], Hq, D), 40, BF), _randn((cu[-1], Hk, D), 41, BF), _randn((cu[-1], Hk, D), 42, BF), _randn((cu[-1], Hq, D), 43, BF)
+    c = torch.tensor(cu, dtype=torch.int32, device=DEV)
+    out, lse = capi.fa_forward_packed(q, k, v, c, c, max(lens), max(lens), is_causal=True)
+    got = capi.fa_backward_packed(do, q, k, v, out, lse, c, c, max(lens), max(lens), is_causal=True)
+    row = lambda t, i: t[cu[i]:cu[i + 1]].transpose(0, 1)[None]
+    for i, n in enumerate(lens):
+        if n:
+            _check_grads([row(t, i) for t in got], _grad_reference(*(row(t, i) for t in (q, k, v, do)), True), BF)

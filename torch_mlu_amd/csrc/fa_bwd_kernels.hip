@@ -4,7 +4,7 @@
 // (torch_mlu/csrc/aten/operators/cnnl/internal/FlashAttention_internal.cpp:449-480) and its descriptor / workspace
 // plumbing (:368-447).
 //
-// Two kernels, no atomics, deterministic:
+// Two kernels (and a merge of partial sums where key blocks are sliced), no atomics, deterministic:
 //   fa_bwd_dq_kernel   — one workgroup = 128 query rows of one (sequence, head), loops over K/V tiles of 64 rows.
 //                        Per lane one query row (as in the forward): S^T = K Q^T, dP^T = V dO^T,
 //                        P^T = exp2(S^T c - LSE), dS^T = P^T o (dP^T - delta), dQ^T += K^T dS^T.
@@ -12,7 +12,8 @@
 //                        second kernel (which then starts its dP accumulators from -delta and needs no rescaling of LSE).
 //   fa_bwd_dkv_kernel  — one workgroup = 128 key rows of one (sequence, kv head), loops over the query heads of the
 //                        GQA group and over Q/dO tiles of 64 rows.  Per lane one key row: S = Q K^T, dP = dO V^T,
-//                        P, dS as above, dV^T += dO^T P, dK^T += Q^T dS.
+//                        P, dS as above, dV^T += dO^T P, dK^T += Q^T dS.  Few key blocks against long chains of heads
+//                        and tiles (GQA): the chains are cut into slices that fa_bwd_dkv_merge_kernel adds up.
 // Both stream their tiles through LDS by global->LDS DMA with one XOR swizzle that is conflict-free for row reads
 // (ds_read_b128, MFMA A operand) and for transposed reads (ds_read_b64_tr_b16) of the same tile.
 // S and dP are recomputed in each kernel (7 matrix products per tile pair instead of 5) in exchange for not needing
@@ -94,7 +95,17 @@ struct BArgs {
   int64_t bias_sb, bias_sh, bias_sq;
   unsigned char* dbias;       // optional gradient of the bias, same addressing
   int64_t dbias_sb, dbias_sh, dbias_sq;
+  // dK/dV of a key block cut into slices (n_slices > 1): slices of at most slice_iters (query head, query tile) steps
+  // leave fp32 partial sums here, which fa_bwd_dkv_merge_kernel adds up
+  float* part;
+  int64_t part_dv;            // floats from the partials of dK to those of dV
+  int32_t n_slices, slice_iters;
 };
+
+// slices of a key block with `niter` steps: as even as possible, none longer than slice_iters
+__device__ __forceinline__ int dkv_slices(const BArgs& a, int niter) {
+  return min(a.n_slices, max(1, (niter + a.slice_iters - 1) / a.slice_iters));
+}
 
 // One swizzle for tiles that are read both by rows (16 lanes = 16 consecutive rows, same logical chunk) and
 // transposed (a half-wave = 4 consecutive rows x 4 consecutive chunks): physical chunk = logical ^ swzU(row).
@@ -555,8 +566,8 @@ __global__ void __launch_bounds__(256, DP > 128 ? 1 : 2) fa_bwd_dq_kernel(const 
 // dK / dV kernel
 // ---------------------------------------------------------------------------------------------------------
 // WHAT selects the outputs: kDK (S, dP, dS, dK), kDV (S, P, dV) or both.  With head_dim 128 both accumulators do not
-// fit the 256 registers that two wavefronts per SIMD leave, so dK and dV run as two launches (S is recomputed once
-// more); with head_dim <= 64 one launch produces both.
+// fit the 256 registers that two wavefronts per SIMD leave, so a workgroup computes dK or dV (S is recomputed once
+// more); with head_dim <= 64 it produces both.
 constexpr int kDK = 1, kDV = 2;
 
 // BIAS: here a lane owns a key column and its registers run over query rows, while the bias is contiguous along keys.
@@ -565,15 +576,16 @@ constexpr int kDK = 1, kDV = 2;
 // (every output is one input times 1.0 plus zeros).  -inf entries are lowered to the most negative finite value
 // first, since -inf * 0 would turn the whole row into NaN; the exponential of either is 0.  A block's loads are issued
 // ahead of its S / dP MFMAs and consumed after them.
+//
+// lid / nwg: this workgroup's number among the nwg that compute WHAT.
 template <typename T, int DP, int WHAT, bool DROP, bool BIAS>
-__global__ void __launch_bounds__(256, DP > 128 ? 1 : 2) fa_bwd_dkv_kernel(const BArgs a) {
+__device__ __forceinline__ void dkv_block(const BArgs& a, unsigned char* smem, int lid, const int nwg) {
   constexpr bool DO_K = (WHAT & kDK) != 0, DO_V = (WHAT & kDV) != 0;
   using IO = TileIO<T, DP>;
   constexpr int CPR = IO::CPR, ROWB = IO::ROWB, TILE = IO::TILE, NI = IO::NI, RPI = IO::RPI, KS = IO::KS, MB = IO::MB;
   constexpr int NV = IO::NV;
   constexpr int BKV = 128, BQ = 64;
   constexpr int VEC = 4 * TILE;  // Q0 Q1 dO0 dO1 | lse[2][64] delta[2][64]
-  extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -582,14 +594,19 @@ __global__ void __launch_bounds__(256, DP > 128 ? 1 : 2) fa_bwd_dkv_kernel(const
 
   // Same dispatch-order reasoning as the dQ kernel.  Causal: the first key blocks are the heavy ones (every query
   // row sees them) and they come first.
-  int lid = blockIdx.x;
-  int pslot, bhk;
-  if (a.cu_q) {
+  int pslot, bhk, slice = 0;
+  if (a.cu_q || a.n_slices > 1) {
+    // sliced: a block's slices one after the other, all (sequence, kv head) pairs of each side by side (with a multiple
+    // of 8 pairs everything that reads one pair's Q and dO runs on one XCD)
     const int nbh = a.batch * a.heads_k;
-    pslot = lid / nbh;
     bhk = lid % nbh;
+    pslot = lid / nbh;
+    if (a.n_slices > 1) {
+      slice = pslot % a.n_slices;
+      pslot /= a.n_slices;
+    }
   } else {
-    const int per = gridDim.x >> 3;
+    const int per = nwg >> 3;
     const int nh = per / a.n_kslot;
     if (a.blockmajor_k && lid < (per << 3) && nh * a.n_kslot == per) {
       const int idx = lid >> 3;
@@ -667,7 +684,15 @@ __global__ void __launch_bounds__(256, DP > 128 ? 1 : 2) fa_bwd_dkv_kernel(const
   if (a.is_causal) jq_begin = max(0, n0 - off) / BQ;
   const int jq_end = (Lq + BQ - 1) / BQ;
   const int nq = max(0, jq_end - jq_begin);
-  const int niter = nq * a.group;  // flattened (query head of the group, query tile)
+  // flattened (query head of the group, query tile); a slice takes steps it0 ... it1 - 1
+  int it0 = 0, it1 = nq * a.group, ns = 1;
+  if (a.n_slices > 1) {
+    ns = dkv_slices(a, it1);
+    if (slice >= ns) return;
+    const int64_t n = it1;
+    it0 = (int)(n * slice / ns);
+    it1 = (int)(n * (slice + 1) / ns);
+  }
 
   // ---- K and V fragments of my key row (B operands) ----
   s16x8 kf[KS], vf[KS];
@@ -725,7 +750,7 @@ __global__ void __launch_bounds__(256, DP > 128 ? 1 : 2) fa_bwd_dkv_kernel(const
       asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off" : : "s"(dst), "v"(src) : "m0");
     }
   };
-  if (niter > 0) issue_iter(0, 0);
+  if (it0 < it1) issue_iter(it0, it0 & 1);
   // The fragments above come from ordinary loads, and the compiler waits for a load at its first use: inside the tile
   // loop that wait (it can only be "every outstanding load") would also cover the next tile's DMA, issued just before,
   // and every tile would start by waiting for its successor.  Using the fragments here puts the wait in front of the
@@ -787,11 +812,11 @@ __global__ void __launch_bounds__(256, DP > 128 ? 1 : 2) fa_bwd_dkv_kernel(const
     for (int i = 0; i < MB; ++i) asm volatile("" : "+a"(dk[i]));
   }
 
-  for (int it = 0; it < niter; ++it) {
+  for (int it = it0; it < it1; ++it) {
     const int buf = it & 1;
     WAIT_VMCNT(0);
     __syncthreads();
-    if (it + 1 < niter) issue_iter(it + 1, buf ^ 1);
+    if (it + 1 < it1) issue_iter(it + 1, buf ^ 1);
     const int jq = jq_begin + it % nq;
     const int qlo = jq * BQ;
     // every (q, kv) of this tile masked for this wavefront: q + off < kv for all pairs
@@ -1046,6 +1071,21 @@ __global__ void __launch_bounds__(256, DP > 128 ? 1 : 2) fa_bwd_dkv_kernel(const
     }
   }
 
+  if (ns > 1) {
+    // a slice's sums stay as the MFMAs left them: 16 bytes per lane, 1 KiB per store instruction
+    const int64_t at = ((((int64_t)pslot * (a.batch * a.heads_k) + bhk) * a.n_slices + slice) * 4 + wave) * (32 * DP) + lane * 4;
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+      for (int v4 = 0; v4 < 4; ++v4) {
+        float* p = a.part + at + (mb * 4 + v4) * 256;
+        if constexpr (DO_K) *(f32x4*)p = f32x4{dk[mb][4 * v4], dk[mb][4 * v4 + 1], dk[mb][4 * v4 + 2], dk[mb][4 * v4 + 3]};
+        if constexpr (DO_V)
+          *(f32x4*)(p + a.part_dv) = f32x4{dv[mb][4 * v4], dv[mb][4 * v4 + 1], dv[mb][4 * v4 + 2], dv[mb][4 * v4 + 3]};
+      }
+    return;
+  }
+
   // dK and dV go out through LDS like the forward's O: staged per wavefront (its 32 key rows, row stride padded by 16
   // bytes), then stored as whole rows.  One staging area per wavefront serves dK, then dV (LDS operations of a
   // wavefront run in order).
@@ -1092,6 +1132,87 @@ __global__ void __launch_bounds__(256, DP > 128 ? 1 : 2) fa_bwd_dkv_kernel(const
   }
 }
 
+// One launch for dK and dV (WHAT = both), so that they share the chip and one tail; two launches left it half empty
+// wherever the kv heads and key blocks made fewer than 512 workgroups.  The two kernels' sum before and the launch now,
+// bf16 causal, head_dim 128: 16 query / 16 kv heads x 2048 rows 104 -> 70 us; 32 / 8 x 4096 722 -> 511; head_dim 256,
+// batch 2, 16 / 8 x 2000 380 -> 253.
+// Where a workgroup computes only one of them (head_dim > 64) the grid holds both kinds in runs of 8 (one per XCD):
+// all of dK and then all of dV, heaviest first (halves), or alternating, which lets the two workgroups of a key block,
+// reading the same Q and dO, meet on one XCD.  Whole backward, alternating / halves, us: batch 8, 32 / 8 x 1500 732 / 706;
+// 16 / 16 x 4096 303 / 287; six packed sequences of up to 4096 rows 1669 / 1627 (head_dim 128, unsliced: halves);
+// head_dim 256, 8 / 8 x 4096 366 / 372; sliced, 28 / 4 x 4096 576 / 587, 8 packed sequences of up to 1500 rows, 16 / 4, 239 / 269.
+template <typename T, int DP, int WHAT, bool DROP, bool BIAS>
+__global__ void __launch_bounds__(256, DP > 128 ? 1 : 2) fa_bwd_dkv_kernel(const BArgs a) {
+  extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
+  if constexpr (DP <= 64 || WHAT != (kDK | kDV)) {
+    dkv_block<T, DP, WHAT, DROP, BIAS>(a, smem, blockIdx.x, gridDim.x);
+  } else {
+    const int nwg = a.batch * a.heads_k * a.n_kslot * a.n_slices;
+    const int runs = (nwg + 7) >> 3;
+    const bool halves = DP == 128 && a.n_slices == 1;
+    int run = (int)blockIdx.x >> 3;
+    const bool is_dv = halves ? run >= runs : (run & 1) != 0;
+    run = halves ? (is_dv ? run - runs : run) : run >> 1;
+    const int lid = run * 8 + (blockIdx.x & 7);
+    if (lid >= nwg) return;
+    if (is_dv) dkv_block<T, DP, kDV, DROP, BIAS>(a, smem, lid, nwg);
+    else dkv_block<T, DP, kDK, DROP, BIAS>(a, smem, lid, nwg);
+  }
+}
+
+// Sum of a key block's slices: one workgroup = 32 key rows (the share of one wavefront of the dK/dV kernel) of dK
+// (blockIdx.y = 0) or dV.  Bound by reading the partials, which mostly still sit in the last-level cache.
+template <typename T, int DP>
+__global__ void __launch_bounds__(256) fa_bwd_dkv_merge_kernel(const BArgs a) {
+  constexpr int BKV = 128, BQ = 64, MB = DP / 32, CPR = DP / 8, ROWB = DP * 2, OSTR = ROWB + 16;
+  __shared__ __attribute__((aligned(16))) unsigned char stage[32 * OSTR];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int g = lane >> 5, c32 = lane & 31;
+  const int nbh = a.batch * a.heads_k;
+  const int part = blockIdx.x & 3, unit = blockIdx.x >> 2;
+  const int bhk = unit % nbh, pslot = unit / nbh;
+  const int hk = bhk % a.heads_k, b = bhk / a.heads_k;
+  const bool is_dv = blockIdx.y != 0;
+  int k0 = 0, Lq = a.seqlen_q, Lk = a.seqlen_k;
+  if (a.cu_q) {
+    Lq = a.cu_q[b + 1] - a.cu_q[b];
+    k0 = a.cu_k[b];
+    Lk = a.cu_k[b + 1] - k0;
+  }
+  const int n0 = pslot * BKV, row0 = n0 + 32 * part;
+  if (row0 >= Lk) return;
+  // the steps of this key block, as the dK/dV kernel counts them
+  const int off = a.causal_tl ? 0 : Lk - Lq;
+  const int jq_begin = a.is_causal ? max(0, n0 - off) / BQ : 0;
+  const int ns = dkv_slices(a, max(0, (Lq + BQ - 1) / BQ - jq_begin) * a.group);
+  if (ns == 1) return;  // written by the dK/dV kernel
+  const float* src = a.part + (is_dv ? a.part_dv : 0) + ((int64_t)unit * a.n_slices * 4 + part) * (32 * DP) + tid * 4;
+  f32x4 sum[MB];
+#pragma unroll
+  for (int i = 0; i < MB; ++i) sum[i] = *(const f32x4*)(src + i * 1024);
+  for (int s = 1; s < ns; ++s) {
+    src += 4 * 32 * DP;
+#pragma unroll
+    for (int i = 0; i < MB; ++i) sum[i] += *(const f32x4*)(src + i * 1024);
+  }
+  const float sc = is_dv ? 1.f : a.scale;
+#pragma unroll
+  for (int i = 0; i < MB; ++i)  // 32-column block i, registers 4 wave ... 4 wave + 3 of it
+    *(u32x2*)(stage + c32 * OSTR + (32 * i + 8 * wave + 4 * g) * 2) =
+        u32x2{Mma<T>::pack2(sum[i][0] * sc, sum[i][1] * sc), Mma<T>::pack2(sum[i][2] * sc, sum[i][3] * sc)};
+  __syncthreads();
+  unsigned char* base = is_dv ? a.dv + (int64_t)hk * a.dv_sh : a.dk + (int64_t)hk * a.dk_sh;
+  const int64_t ss = is_dv ? a.dv_ss : a.dk_ss;
+  if (!a.cu_q) base += (int64_t)b * (is_dv ? a.dv_sb : a.dk_sb);
+  base += (int64_t)(k0 + row0) * ss;
+#pragma unroll
+  for (int i = 0; i < 32 * CPR / 256; ++i) {
+    const int r = (i * 256 + tid) / CPR, ch = (i * 256 + tid) % CPR;
+    if (r < Lk - row0 && ch * 8 < a.head_dim) *(u32x4*)(base + (int64_t)r * ss + ch * 16) = *(const u32x4*)(stage + r * OSTR + ch * 16);
+  }
+}
+
 // ---------------------------------------------------------------------------------------------------------
 // Host side
 // ---------------------------------------------------------------------------------------------------------
@@ -1104,7 +1225,6 @@ template <typename T, int DP, bool DROP, bool BIAS>
 int bwd_launch(const BArgs& a, hipStream_t st) {
   constexpr int lds_dq = 4 * 64 * DP * 2;
   constexpr int lds_dkv = 4 * 64 * DP * 2 + 4 * 256;
-  constexpr bool split = DP > 64;  // head_dim 128: dK and dV as two launches
   constexpr auto kq = fa_bwd_dq_kernel<T, DP, DROP, BIAS ? 1 : 0>;
   // the dQ kernel can fetch 16-byte pieces of bias rows by DMA when every row starts 16-byte aligned and no piece
   // straddles the end of a row
@@ -1114,13 +1234,17 @@ int bwd_launch(const BArgs& a, hipStream_t st) {
   const bool staged = can_stage && !a.cu_q && a.seqlen_k % 8 == 0 && (uintptr_t)a.bias % 16 == 0 && a.bias_sb % 16 == 0 &&
                       a.bias_sh % 16 == 0 && a.bias_sq % 16 == 0 && a.bias_sq <= kMaxRowStrideBytes;
   if (staged && !ensure_dynamic_lds<kq2>(lds_dq2)) return FA_ERR_LAUNCH;
+  // with dropout or a bias the merged dK / dV kernel of head_dim > 64 would spill: two launches
+  constexpr bool split = DP > 64 && (DROP || BIAS);
   constexpr auto kkv = fa_bwd_dkv_kernel<T, DP, split ? kDK : (kDK | kDV), DROP, BIAS>;
-  constexpr auto kv2 = fa_bwd_dkv_kernel<T, DP, kDV, DROP, BIAS>;
+  constexpr auto kv2 = fa_bwd_dkv_kernel<T, DP, split ? kDV : (kDK | kDV), DROP, BIAS>;
   if (!ensure_dynamic_lds<kq>(lds_dq) || !ensure_dynamic_lds<kkv>(lds_dkv) || (split && !ensure_dynamic_lds<kv2>(lds_dkv)))
     return FA_ERR_LAUNCH;
   const int64_t gq = (int64_t)a.batch * a.heads_q * a.n_qslot;
-  const int64_t gk = (int64_t)a.batch * a.heads_k * a.n_kslot;
-  if (gq > 0x7fffffffLL || gk > 0x7fffffffLL) return FA_ERR_UNSUPPORTED;
+  const int64_t units = (int64_t)a.batch * a.heads_k * a.n_kslot;
+  // head_dim > 64, one launch: a workgroup each for dK and dV, in runs of 8
+  const int64_t gk = (DP > 64 && !split) ? (units * a.n_slices + 7) / 8 * 16 : units * a.n_slices;
+  if (gq > 0x7fffffffLL || gk > 0x7fffffffLL || units * 4 > 0x7fffffffLL) return FA_ERR_UNSUPPORTED;
   if (gq > 0) {
     if (staged) hipLaunchKernelGGL(kq2, dim3((unsigned)gq), dim3(256), lds_dq2, st, a);
     else hipLaunchKernelGGL(kq, dim3((unsigned)gq), dim3(256), lds_dq, st, a);
@@ -1131,6 +1255,10 @@ int bwd_launch(const BArgs& a, hipStream_t st) {
     if (hipGetLastError() != hipSuccess) return FA_ERR_LAUNCH;
     if (split) {
       hipLaunchKernelGGL(kv2, dim3((unsigned)gk), dim3(256), lds_dkv, st, a);
+      if (hipGetLastError() != hipSuccess) return FA_ERR_LAUNCH;
+    }
+    if (a.n_slices > 1) {
+      hipLaunchKernelGGL((fa_bwd_dkv_merge_kernel<T, DP>), dim3((unsigned)(units * 4), 2), dim3(256), 0, st, a);
       if (hipGetLastError() != hipSuccess) return FA_ERR_LAUNCH;
     }
   }
@@ -1174,6 +1302,10 @@ int fa_bwd_launch(const fa_bwd_params* p, void* workspace, size_t workspace_byte
   a.dq = (unsigned char*)p->dq; a.dk = (unsigned char*)p->dk; a.dv = (unsigned char*)p->dv;
   a.delta = (float*)workspace;
   a.lse2 = (float*)((unsigned char*)workspace + bwd_ws_plane(p));
+  const host::BwdSlices sl = host::bwd_slices(p);
+  a.n_slices = sl.count; a.slice_iters = sl.iters;
+  a.part = (float*)((unsigned char*)workspace + 2 * bwd_ws_plane(p));
+  a.part_dv = (int64_t)(sl.bytes / 8);
   a.cu_q = p->cu_seqlens_q; a.cu_k = p->cu_seqlens_k;
   a.q_sb = p->q_stride_b * 2; a.q_ss = p->q_stride_s * 2; a.q_sh = p->q_stride_h * 2;
   a.k_sb = p->k_stride_b * 2; a.k_ss = p->k_stride_s * 2; a.k_sh = p->k_stride_h * 2;

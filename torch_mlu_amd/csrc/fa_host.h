@@ -237,7 +237,51 @@ inline size_t bwd_ws_plane(const fa_bwd_params* p) {
   const size_t rows = p->cu_seqlens_q ? (size_t)p->total_q : (size_t)p->batch * p->seqlen_q;
   return (rows * p->heads_q * 4 + 15) & ~(size_t)15;
 }
-inline size_t bwd_ws_bytes(const fa_bwd_params* p) { return 2 * bwd_ws_plane(p); }
+// Slices of a key block's dK / dV.  A key block's workgroup walks the query tiles of all heads of its group one after
+// the other, and one workgroup already keeps its CU's matrix cores as busy as two do, so a launch takes at least as long
+// as its longest block alone: a group of 7 heads over 4096 rows is 448 steps of 1.7 us whatever the rest of the chip
+// does.  Where that is more than the whole work spread over the 256 CUs, the blocks are cut into slices whose fp32
+// partial sums a second kernel adds up.  A step costs 1.7 us of a CU for dK and 1.25 for dV (one workgroup each; at
+// head_dim 64 one workgroup does both), a slice's partials, start and share of the merge about as much as 6 steps and
+// the extra launch 10.  Whole backward, bf16, causal, unsliced -> sliced, us: 28 query / 4 kv heads, head_dim 128, 4096
+// rows 882 -> 575, 700 rows 145 -> 60; 32 / 8, 2048 rows 272 -> 195, 4096 rows 642 -> 607; batch 4, 16 / 4, head_dim 64,
+// 2048 rows 225 -> 165; 8 packed sequences of 187 ... 1500 rows, 16 / 4, 250 -> 232.  On the other side of the line:
+// 16 / 16, 2048 rows 113 -> 133; 8 / 8, 4096 rows 209 -> 222; batch 2, 16 / 8, head_dim 256, 2000 rows 331 -> 423.
+struct BwdSlices {
+  int32_t count;  // most slices of a key block
+  int32_t iters;  // most steps (query head of the group, 64-row query tile) of a slice
+  size_t bytes;   // fp32 partial sums of dK, then of dV
+};
+inline BwdSlices bwd_slices(const fa_bwd_params* p) {
+  BwdSlices r = {1, 0x7fffffff, 0};
+  const int64_t group = p->heads_q / p->heads_k;
+  const int64_t units = (int64_t)p->batch * p->heads_k * ((p->seqlen_k + 127) / 128);
+  const int64_t longest = group * ((p->seqlen_q + 63) / 64);
+  if (units == 0 || longest == 0) return r;
+  // steps of all blocks; packed lengths are known on the device only, and sum(n^2) lies between total^2 / batch (equal
+  // lengths) and total x longest: the geometric mean of the two, with a margin for being an estimate
+  double total = (double)units * (double)longest * (p->is_causal != FA_MASK_NONE ? 0.5 : 1.0), margin = 1.0;
+  if (p->cu_seqlens_q) {
+    const double fill = (double)p->total_q / ((double)p->batch * p->seqlen_q);
+    if (fill < 1.0) total *= fill * sqrt(fill);
+    margin = 1.25;
+  }
+  const double spread = total / 256.0 * (p->head_dim <= 64 ? 1.2 : 1.75);
+  if ((double)longest <= margin * (spread + 10.0)) return r;
+  // about four slices per CU (of each kind), of 16 steps at least
+  int64_t want = (int64_t)(total / 1024.0);
+  if (want < 16) want = 16;
+  int64_t n = (longest + want - 1) / want;
+  if (n > FA_MAX_SPLITS) n = FA_MAX_SPLITS;
+  const int64_t slot = (int64_t)128 * padded_dim(p->head_dim) * 4 * 2;
+  while (n > 1 && units > (1LL << 30) / (slot * n)) --n;
+  if (n <= 1) return r;
+  r.count = (int32_t)n;
+  r.iters = (int32_t)((longest + n - 1) / n);
+  r.bytes = (size_t)(units * n * slot);
+  return r;
+}
+inline size_t bwd_ws_bytes(const fa_bwd_params* p) { return 2 * bwd_ws_plane(p) + bwd_slices(p).bytes; }
 
 }  // namespace host
 }  // namespace fa
