@@ -457,7 +457,7 @@ __global__ void __launch_bounds__(256, DP > 128 ? 1 : 2) fa_bwd_dq_kernel(const 
         if (32 + e > lim) s1[v] = gone;
       }
     }
-    const uint32_t drop_tile = DROP ? (drop_row ^ drop_col_term((uint32_t)(j * (BN / 2) + 2 * g))) : 0u;
+    const uint32_t drop_tile = DROP ? (drop_row ^ drop_col_term((uint32_t)(j * (BN / 2) + 2 * g)) ^ (uint32_t)(row & 1)) : 0u;
     s16x8 dsb[4];
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
@@ -466,14 +466,16 @@ __global__ void __launch_bounds__(256, DP > 128 ? 1 : 2) fa_bwd_dq_kernel(const 
         braw[4 * (t >> 1) + 2 * (t & 1) + 1] = *(const u32x2*)(smem + (baddr ^ ((4 * (t >> 1) + 2 * (t & 1) + 1) * 16)));
       }
       u32x4 w;
+      uint32_t words[4];
+      if constexpr (DROP) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+          drop_words(drop_tile ^ (uint32_t)(16 * (t >> 1) + 8 * (t & 1) + 4 * i), drop_key2, words[2 * i], words[2 * i + 1]);
+      }
 #pragma unroll
       for (int e2 = 0; e2 < 4; ++e2) {
         float ds[2];
-        uint32_t word = 0;
-        if constexpr (DROP) {
-          const int v0 = 8 * (t & 1) + 2 * e2;
-          word = drop_word(drop_tile ^ (uint32_t)(16 * (t >> 1) + 4 * (v0 >> 2) + ((v0 & 3) >> 1)), drop_key2) >> drop_sh;
-        }
+        const uint32_t word = DROP ? words[e2] >> drop_sh : 0u;
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
           const int v = 8 * (t & 1) + 2 * e2 + u;
@@ -826,7 +828,8 @@ __device__ __forceinline__ void dkv_block(const BArgs& a, unsigned char* smem, i
     uint32_t drop_tile = 0, drop_key2 = 0;
     if constexpr (DROP) {
       const DropKeys dk = drop_head_keys(drop_seed, drop_offset, (uint32_t)(b * a.heads_q + hk * a.group + it / nq));
-      drop_tile = dk.k1 ^ drop_col ^ drop_row_term((uint32_t)(qlo / 2 + 2 * g));
+      // (the odd lane of a column pair hashes the odd row pairs, see drop_words)
+      drop_tile = dk.k1 ^ drop_col ^ drop_row_term((uint32_t)(qlo / 2 + 2 * g)) ^ ((uint32_t)(kvrow & 1) << 16);
       drop_key2 = dk.k2;
     }
 
@@ -902,14 +905,19 @@ __device__ __forceinline__ void dkv_block(const BArgs& a, unsigned char* smem, i
 #pragma unroll
       for (int tt = 0; tt < 4; ++tt) {  // chunk tt: rows 16 tt .. 16 tt + 15 = block tt / 2, half tt % 2
         u32x4 wp;
+        uint32_t words[4];
+        if constexpr (DROP) {
+#pragma unroll
+          for (int i = 0; i < 2; ++i)
+            drop_words(drop_tile ^ ((uint32_t)(16 * (tt >> 1) + 8 * (tt & 1) + 4 * i) << 16), drop_key2, words[2 * i], words[2 * i + 1]);
+        }
 #pragma unroll
         for (int e2 = 0; e2 < 4; ++e2) {
           const int qbk = tt >> 1, v = 8 * (tt & 1) + 2 * e2;
           const float l0 = lv[qbk][v >> 2][v & 3], l1 = lv[qbk][v >> 2][(v & 3) + 1];
           float p0 = fast_exp2(s2[qbk][v] * c - l0), p1 = fast_exp2(s2[qbk][v + 1] * c - l1);
           if constexpr (DROP) {
-            const uint32_t rp_const = 16 * qbk + 4 * (v >> 2) + ((v & 3) >> 1);
-            const uint32_t word = drop_word(drop_tile ^ (rp_const << 16), drop_key2) >> drop_sh;
+            const uint32_t word = words[e2] >> drop_sh;
             p0 = ((word & 0xffu) <= a.drop_thr) ? p0 * a.drop_rp : 0.f;
             p1 = (((word >> 16) & 0xffu) <= a.drop_thr) ? p1 * a.drop_rp : 0.f;
           }
@@ -1008,6 +1016,12 @@ __device__ __forceinline__ void dkv_block(const BArgs& a, unsigned char* smem, i
             if constexpr (DO_K && !DELTA_INIT) dl[q4] = *(const f32x4*)(del_t + 32 * qbk + 8 * q4 + 4 * g);
           }
         }
+        uint32_t words[4];
+        if constexpr (DROP) {
+#pragma unroll
+          for (int i = 0; i < 2; ++i)
+            drop_words(drop_tile ^ ((uint32_t)(16 * qbk + 8 * t + 4 * i) << 16), drop_key2, words[2 * i], words[2 * i + 1]);
+        }
 #pragma unroll
         for (int e2 = 0; e2 < 4; ++e2) {
           const int v = 8 * t + 2 * e2;  // v, v + 1: consecutive query rows
@@ -1023,8 +1037,7 @@ __device__ __forceinline__ void dkv_block(const BArgs& a, unsigned char* smem, i
           float dp0 = DO_K ? dp[v] : 0.f, dp1 = DO_K ? dp[v + 1] : 0.f;
           float pv0 = p0, pv1 = p1;  // what multiplies dO in dV: P o M / keep
           if constexpr (DROP) {
-            const uint32_t rp_const = 16 * qbk + 4 * (v >> 2) + ((v & 3) >> 1);
-            const uint32_t word = drop_word(drop_tile ^ (rp_const << 16), drop_key2) >> drop_sh;
+            const uint32_t word = words[e2] >> drop_sh;
             const bool k0 = (word & 0xffu) <= a.drop_thr, k1 = ((word >> 16) & 0xffu) <= a.drop_thr;
             pv0 = k0 ? p0 * a.drop_rp : 0.f;
             pv1 = k1 ? p1 * a.drop_rp : 0.f;

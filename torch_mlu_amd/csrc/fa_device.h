@@ -183,6 +183,15 @@ __device__ __forceinline__ uint32_t drop_word(uint32_t counter, uint32_t key2) {
   h ^= h >> 16;
   return h;
 }
+// In the score layouts of the tile and backward kernels two neighbouring lanes own the two rows (or columns) of a patch
+// and need the same words, so each hashes half of them and passes them on: `counter`, the even lane's, and the odd
+// lane's, whose bit differs, give the words of both.  A word costs two 32-bit multiplications at a quarter of the
+// vector rate and eight plain instructions, the exchange two moves a pair.
+__device__ __forceinline__ void drop_words(uint32_t counter, uint32_t key2, uint32_t& even, uint32_t& odd) {
+  const int h = (int)drop_word(counter, key2);
+  even = (uint32_t)__builtin_amdgcn_mov_dpp(h, 0xa0, 0xf, 0xf, true);  // quad_perm [0, 0, 2, 2]
+  odd = (uint32_t)__builtin_amdgcn_mov_dpp(h, 0xf5, 0xf, 0xf, true);   // quad_perm [1, 1, 3, 3]
+}
 // keys of one (sequence b, query head h) of one call: bh = b * heads_q + h
 struct DropKeys {
   uint32_t k1, k2;

@@ -588,7 +588,8 @@ __global__ void __launch_bounds__(256, MINB) fa_tile_kernel(const KArgs a) {
     const float mc = mc_run;  // m_run c, kept alongside m_run (0 while no key has been seen)
     // dropout: counter of a patch = key ^ row term ^ column term; the column pair of this lane's groups is
     // 32 j + 2 g + a compile-time constant with disjoint bits
-    const uint32_t drop_tile = DROP ? (drop_row ^ drop_col_term((uint32_t)(j * (BN / 2) + 2 * g))) : 0u;
+    // (the odd lane of a row pair hashes the odd column pairs, see drop_words)
+    const uint32_t drop_tile = DROP ? (drop_row ^ drop_col_term((uint32_t)(j * (BN / 2) + 2 * g)) ^ (uint32_t)(row & 1)) : 0u;
 
     // ---- per 16-key chunk t: P = exp2(S c - m c), row sums, P^T as B operand, O^T += V^T P^T.  The V^T fragments
     //      of chunk t + 1 are fetched while chunk t's MFMAs run. ----
@@ -608,6 +609,12 @@ __global__ void __launch_bounds__(256, MINB) fa_tile_kernel(const KArgs a) {
         for (int mb = 0; mb < MB; ++mb) va[(t + 1) & 1][mb] = vfrag(mb, t + 1);
       }
       u32x4 w;
+      uint32_t words[4];  // patch words of the chunk's column pairs: keys j BN + 32 (t >> 1) + 8 (v >> 2) + 4 g + (v & 3), + 1
+      if constexpr (DROP) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+          drop_words(drop_tile ^ (uint32_t)(16 * (t >> 1) + 8 * (t & 1) + 4 * i), drop_key2, words[2 * i], words[2 * i + 1]);
+      }
 #pragma unroll
       for (int e2 = 0; e2 < 4; ++e2) {
         const int v = 8 * (t & 1) + 2 * e2;
@@ -617,9 +624,7 @@ __global__ void __launch_bounds__(256, MINB) fa_tile_kernel(const KArgs a) {
         constexpr bool sum_packed = Mma<T>::kSumPacked && !DROP;
         if constexpr (!sum_packed) rs += p0 + p1;
         if constexpr (DROP) {
-          // keys j BN + 32 (t >> 1) + 8 (v >> 2) + 4 g + (v & 3), + 1: one column pair, one patch word
-          const uint32_t cp_const = 16 * (t >> 1) + 4 * (v >> 2) + ((v & 3) >> 1);
-          const uint32_t word_full = drop_word(drop_tile ^ cp_const, drop_key2);
+          const uint32_t word_full = words[e2];
           if constexpr (!DMASK) {
             // The pair's two bytes go to the low bytes of the two 16-bit halves (one v_perm_b32), threshold minus
             // byte is negative exactly where the element is dropped, and its sign, spread over the half by an
