@@ -108,8 +108,8 @@ typedef struct fa_bwd_params {
 /* Host-only validation: FA_OK or a negative code (FA_ERR_UNSUPPORTED for head_dim > 256). */
 FA_API int fa_bwd_validate(const fa_bwd_params* p);
 
-/* Bytes of device scratch fa_bwd_launch needs (-rowsum(dO o O) and LSE log2(e), two fp32 per query row and head);
-   0 if invalid. */
+/* Bytes of device scratch fa_bwd_launch needs (-rowsum(dO o O) and LSE log2(e), two fp32 per query row and head; and,
+   where the work of a key block is cut into slices, the slices' fp32 sums of dK and dV, at most 1 GiB); 0 if invalid. */
 FA_API size_t fa_bwd_workspace_bytes(const fa_bwd_params* p);
 
 /* Enqueue the backward pass on `stream`; `workspace` must hold fa_bwd_workspace_bytes(p) bytes, 16-byte aligned. */
