@@ -157,6 +157,9 @@ __device__ __forceinline__ float max3d(float a, float b, float c, float after) {
   return r;
 }
 
+// memory that no one writes while a kernel runs: a load at a wavefront-uniform address is a scalar one
+typedef const __attribute__((address_space(4))) int32_t* ConstI32Ptr;
+
 // ---- dropout ---------------------------------------------------------------------------------------------
 // One 32-bit word per 2 x 2 patch of the attention matrix of one (sequence, query head); element (row, col) keeps its
 // probability iff byte 2 (row & 1) + (col & 1) of the patch's word is <= the threshold.  The word is a murmur3

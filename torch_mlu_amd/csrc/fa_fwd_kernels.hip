@@ -233,10 +233,10 @@ __global__ void __launch_bounds__(256, MINB) fa_tile_kernel(const KArgs a) {
   struct PageRef {
     int pg0, pg1, ro0, ro1;
   };
-  const int32_t* tbl = nullptr;
+  ConstI32Ptr tbl = nullptr;  // scalar loads, see fa_splitkv_kernel
   int psz = 32, lk_idx = 0, lk_ro = 0, lk_max = 0;
   if constexpr (PAGED) {
-    tbl = a.block_table + (int64_t)b * a.bt_stride;
+    tbl = (ConstI32Ptr)(uintptr_t)(a.block_table + (int64_t)b * a.bt_stride);
     psz = a.page_size;
     lk_max = max(last_k, 0) / psz;  // the last entry that belongs to this sequence's keys
   }
@@ -251,8 +251,8 @@ __global__ void __launch_bounds__(256, MINB) fa_tile_kernel(const KArgs a) {
       ++i1;
     }
     // (wavefront-uniform by construction; said so, since the DMA's base address must live in scalar registers)
-    const PageRef r{__builtin_amdgcn_readfirstlane(tbl[min(lk_idx, lk_max)]),
-                    __builtin_amdgcn_readfirstlane(tbl[min(i1, lk_max)]), __builtin_amdgcn_readfirstlane(lk_ro),
+    const PageRef r{tbl[__builtin_amdgcn_readfirstlane(min(lk_idx, lk_max))],
+                    tbl[__builtin_amdgcn_readfirstlane(min(i1, lk_max))], __builtin_amdgcn_readfirstlane(lk_ro),
                     __builtin_amdgcn_readfirstlane(o1)};
     lk_ro += BN;
     while (lk_ro >= psz) {
@@ -866,8 +866,9 @@ __global__ void __launch_bounds__(NW * 64, 1) fa_splitkv_kernel(const KArgs a) {
 
   // Paged cache: a 32-row block lies inside one page (page_size is a multiple of 32), so the page is one scalar
   // table entry per block, requested a block ahead of its use; (pg_idx, pg_in) walks (entry, block in the page) without
-  // a division.
-  const int32_t* tbl = a.block_table ? a.block_table + (int64_t)b * a.bt_stride : nullptr;
+  // a division.  A scalar load has to be asked for (the table does not change under the kernel): read as ordinary memory
+  // an entry came by a vector load, whose wait also covered the two blocks requested before it.
+  ConstI32Ptr tbl = a.block_table ? (ConstI32Ptr)(uintptr_t)(a.block_table + (int64_t)b * a.bt_stride) : nullptr;
   const int bpp = tbl ? a.page_size >> 5 : 1;  // blocks per page
   int pg_idx = 0, pg_in = 0;
   if (tbl) {
@@ -876,7 +877,7 @@ __global__ void __launch_bounds__(NW * 64, 1) fa_splitkv_kernel(const KArgs a) {
     kp = a.k + (int64_t)hk * a.k_sh;
     vp = a.v + (int64_t)hk * a.v_sh;
   }
-  auto lookup = [&](bool exists) { return tbl && exists ? __builtin_amdgcn_readfirstlane(tbl[pg_idx]) : 0; };
+  auto lookup = [&](bool exists) -> int { return tbl && exists ? tbl[pg_idx] : 0; };
   // fetch block blk (this wavefront's next one) into `stage`; page: its table entry
   auto issue_block = [&](int blk, int stage, int page) {
     const unsigned dst = ring + stage * Cfg::STAGE;
@@ -1291,10 +1292,12 @@ int launch_splitkv(const KArgs& a, hipStream_t st) {
 
 // Sequences of one length: four wavefronts and most of a CU's LDS per workgroup, whose slices are equal and in step
 // (6.0 TB/s at B = 64, 8192 keys; two wavefronts: 5.6).  Ragged lengths: half the size, so that two workgroups share a CU
-// and one's start and merge are covered by the other's loads (32 sequences of 1024 ... 4096 keys: 73 against 80 us).
+// and one's start and merge are covered by the other's loads (512 units of up to 512 keys: 21 against 24 us), except where
+// there is one workgroup per CU at most, which then needs all of the CU's loads in flight (212 units of up to 1728 keys: 29
+// against 35 us).
 template <typename T, bool DROP>
 int dispatch_splitkv(const KArgs& a, int dp, hipStream_t st) {
-  const bool ragged = a.seqused_k || a.cu_q;
+  const bool ragged = (a.seqused_k || a.cu_q) && (a.n_splits > 1 || (int64_t)a.batch * a.heads_k > 256);
   if (dp == 64) return ragged ? launch_splitkv<T, 64, 2, DROP>(a, st) : launch_splitkv<T, 64, 4, DROP>(a, st);
   if (dp == 128) return ragged ? launch_splitkv<T, 128, 2, DROP>(a, st) : launch_splitkv<T, 128, 4, DROP>(a, st);
   return launch_splitkv<T, 256, 2, DROP>(a, st);

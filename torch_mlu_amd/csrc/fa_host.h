@@ -123,13 +123,16 @@ inline void plan(const fa_fwd_params* p, int* kernel, int* splits) {
         // Ragged lengths, known on the device only: seqlen_k is the longest possible one, and a sequence's slices are
         // cut from its own length.  One round of the 512 resident (half-size) workgroups is wanted while slices of the
         // longest keep 128 rows, and up to three, to even out what the dispatcher hands the CUs, while they keep 512.
-        // Measured on 7 ... 64 sequences of 2k ... 8k keys: within 3 % of the best count.
+        // Where the units alone come near one per CU, slices and their merge have to buy more: two whole rounds of 640
+        // rows, or none.  Measured on 2 ... 64 paged sequences of up to 512 ... 16k keys: within 5 % of the best count
+        // (212 units of 1728 keys: one slice 29 us, three 36; 256 of 2048: 36, two 41; 256 of 4096: 63, six 61).
         auto most = [&](int64_t wgs, int64_t rows) {
           const int64_t fill = (wgs + units - 1) / units, cap = p->seqlen_k / rows;
           return fill < cap ? fill : cap;
         };
-        const int64_t one = most(512, 128), three = most(1536, 512);
+        const int64_t one = most(512, 128), three = most(1536, units >= 192 ? 640 : 512);
         int64_t n = one > three ? one : three;
+        if (units >= 192) n = units * three >= 1024 ? three : 1;
         if (n > 8) n &= ~(int64_t)3;
         ns = (int)(n < 1 ? 1 : (n > FA_MAX_SPLITS ? FA_MAX_SPLITS : n));
       } else {
