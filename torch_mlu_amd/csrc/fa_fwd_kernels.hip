@@ -132,7 +132,7 @@ __global__ void __launch_bounds__(256, MINB) fa_tile_kernel(const KArgs a) {
     const int nbh = a.batch * a.heads_q;
     pslot = lid / nbh;
     bh = lid % nbh;
-  } else if (a.lpt) {
+  } else if (!BIAS && a.lpt) {
     // Causal, too few blocks to pair: the last (heaviest) blocks of all heads first.  A grid of at most two workgroups
     // per CU is placed all at once, workgroup i on the CU of workgroup i - 256, so its second half runs backwards and
     // every CU gets a heavy and a light block.  With 8 k heads a head's blocks still meet on one XCD.
