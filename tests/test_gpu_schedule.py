@@ -55,6 +55,28 @@ def test_merge_of_slices(D, Sq):
 
 
 @pytest.mark.parametrize("D", [64, 128, 256])
+@pytest.mark.parametrize("kernel,B,Hq,Hk,Sq", [
+    (capi.FA_KERNEL_TILE, 2, 4, 2, 130),      # 1040 rows: four wavefronts merge a row
+    (capi.FA_KERNEL_TILE, 2, 4, 2, 300),      # 2400 rows: one
+    (capi.FA_KERNEL_SPLITKV, 2, 8, 2, 2),     # 32
+    (capi.FA_KERNEL_SPLITKV, 64, 32, 2, 1),   # 2048
+])
+def test_merge_keeps_infinities_of_the_last_slice(D, kernel, B, Hq, Hk, Sq):
+    """Every row sees every key, so an infinite value of V makes its column infinite and leaves the others alone, in the
+    last of the merged slices (whose partials are loaded once more in the place of slices that do not exist) too."""
+    Sk = 80 * (64 if kernel == capi.FA_KERNEL_TILE else 32)  # blocks that 2, 5, 8 and 16 slices share evenly
+    q, k, v = _randn((B, Hq, Sq, D), 50, HF), _randn((B, Hk, Sk, D), 51, HF), _randn((B, Hk, Sk, D), 52, HF)
+    v[:, :, Sk - 7, 5] = float("inf")
+    v[:, :, Sk - 3, D - 2] = float("-inf")
+    whole = capi.fa_forward_dense(q, k, v, kernel=kernel, num_splits=1)[0]
+    assert (whole[..., 5] == float("inf")).all() and (whole[..., D - 2] == float("-inf")).all()
+    for ns in (2, 5, 8, 16):
+        out = capi.fa_forward_dense(q, k, v, kernel=kernel, num_splits=ns)[0]
+        assert torch.equal(out.isinf(), whole.isinf()) and torch.equal(out[whole.isinf()], whole[whole.isinf()])
+        assert (out - whole).masked_fill(whole.isinf(), 0.0).abs().max().item() <= OUT_TOL[HF]  # (a NaN fails this)
+
+
+@pytest.mark.parametrize("D", [64, 128, 256])
 @pytest.mark.parametrize("used", [None, 31, 32, 33, 127, 128, 129, 255, 257, 1000])
 def test_decode_slices_around_the_blocks_of_a_wavefront(D, used):
     """Slices of 0, 1, 2 and more 32-row blocks per wavefront, four wavefronts a workgroup (equal lengths) and two

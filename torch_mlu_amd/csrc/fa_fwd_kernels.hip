@@ -1154,12 +1154,14 @@ __global__ void __launch_bounds__(256) fa_merge_rows_kernel(const KArgs a) {
   for (int o = 32; o >= 1; o >>= 1) lsum += __shfl_xor(lsum, o);
   f32x4 acc = {0.f, 0.f, 0.f, 0.f};
   for (;;) {
-    // a slice that saw no key leaves zeros (the tile kernel) or finite partial sums; its factor is 0 either way
+    // A slice that saw no key leaves zeros (the tile kernel) or finite partial sums; its factor is 0 either way.  What was
+    // loaded in the place of a slice that does not exist is the last slice once more and must not enter the sum at all,
+    // not even times 0: it is infinite where V is.
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int s = s0 + u * s_step;
       const float f = __shfl(scl, min(s, 63));
-      acc += x[u] * (s < ns ? f : 0.f);
+      if (s < ns) acc += x[u] * f;
     }
     s0 += U * s_step;
     if (s0 - sub - wr * spw >= ns) break;  // (uniform over the wavefronts of the row)
