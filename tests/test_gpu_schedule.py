@@ -36,14 +36,35 @@ def _check(q, k, v, causal, **kw):
 @pytest.mark.parametrize("B,H,S", [
     (1, 33, 1024),   # 264 blocks: a few more than one per CU, heads do not divide 256
     (1, 64, 640),    # 320
-    (2, 64, 500),    # 512: two per CU, the second half runs backwards
+    (2, 64, 500),    # 512: two per CU, the second half runs backwards at head_dim 128
     (1, 65, 1000),   # 520: more than two per CU
     (2, 62, 1000),   # 992 blocks = 496 pairs: one pair per resident workgroup
     (1, 520, 130),   # 1040 blocks, two per head
 ])
-def test_every_causal_block_is_computed(B, H, S):
-    q, k, v = _randn((B, H, S, 64), 1, HF), _randn((B, H, S, 64), 2, HF), _randn((B, H, S, 64), 3, HF)
+@pytest.mark.parametrize("D", [64, 128, 256])
+def test_every_causal_block_is_computed(D, B, H, S):
+    q, k, v = _randn((B, H, S, D), 1, HF), _randn((B, H, S, D), 2, HF), _randn((B, H, S, D), 3, HF)
     _check(q, k, v, True)
+
+
+@pytest.mark.parametrize("D", [64, 128, 256])
+@pytest.mark.parametrize("B,Hq,Hk,S", [(2, 64, 16, 500), (1, 36, 4, 1000), (4, 32, 8, 1000)])   # 512, 288, 1024 blocks
+def test_every_causal_block_is_computed_with_dropout_and_grouped_heads(D, B, Hq, Hk, S):
+    q, k, v = _randn((B, Hq, S, D), 1, HF), _randn((B, Hk, S, D), 2, HF), _randn((B, Hk, S, D), 3, HF)
+    _check(q, k, v, True)
+    kw = dict(is_causal=True, dropout_p=0.25, philox_seed=3, philox_offset=8)
+    mask = torch.zeros((B, Hq, S, S), dtype=HF, device=DEV)
+    capi.fa_forward_dense(q, k, v, dropout_mask=mask, **kw)
+    out, lse = capi.fa_forward_dense(q, k, v, **kw)
+    s = q.float() @ k.float().repeat_interleave(Hq // Hk, 1).transpose(2, 3).contiguous() / math.sqrt(D)
+    s.masked_fill_(torch.ones(S, S, dtype=torch.bool, device=DEV).triu(1), float("-inf"))
+    want_l = torch.logsumexp(s, -1)
+    keep = (math.floor(0.75 * 255) + 1) / 256
+    want = (torch.exp(s - want_l[..., None]) * (mask > 0) / keep) @ v.float().repeat_interleave(Hq // Hk, 1)
+    assert torch.equal(mask != 0, (s > float("-inf")))
+    # the bar of the dropout tests: two units in the last place of the largest value, which the first rows' reach
+    assert (out.float() - want).abs().max().item() <= 2 * 2.0 ** -11 * max(1.0, want.abs().max().item())
+    assert (lse - want_l).abs().max().item() <= LSE_TOL
 
 
 @pytest.mark.parametrize("D", [64, 72, 128, 256])

@@ -27,7 +27,7 @@ struct KArgs {
   int32_t seqlen_q, seqlen_k, head_dim;
   int32_t n_mblk;     // tile kernels: workgroups per (sequence, head)
   int32_t pair;       // tile kernel: a workgroup owns query blocks p and n-1-p of its sequence
-  int32_t lpt;        // tile kernel, dense causal, unpaired: heaviest blocks of all heads first
+  int32_t lpt;        // tile kernel, dense causal, unpaired: heaviest blocks of all heads first (2: second half backwards)
   int32_t hgroup;     // tile kernel with a bias that is shared by all heads: heads whose workgroups are interleaved
   int32_t n_splits;   // split-KV kernel; tile kernel: slices of the key range per query block (1 = none)
   int32_t is_causal;

@@ -133,11 +133,11 @@ __global__ void __launch_bounds__(256, MINB) fa_tile_kernel(const KArgs a) {
     pslot = lid / nbh;
     bh = lid % nbh;
   } else if (!BIAS && a.lpt) {
-    // Causal, too few blocks to pair: the last (heaviest) blocks of all heads first.  A grid of at most two workgroups
-    // per CU is placed all at once, workgroup i on the CU of workgroup i - 256, so its second half runs backwards and
-    // every CU gets a heavy and a light block.  With 8 k heads a head's blocks still meet on one XCD.
+    // Causal, too few blocks to pair: the last (heaviest) blocks of all heads first.  lpt == 2: a grid of at most two
+    // workgroups per CU that is placed all at once, workgroup i on the CU of workgroup i - 256, runs its second half
+    // backwards, so that every CU gets a heavy and a light block.  With 8 k heads a head's blocks still meet on one XCD.
     const int nbh = a.batch * a.heads_q, total = gridDim.x;
-    const bool back = total <= 512 && lid >= 256;
+    const bool back = a.lpt == 2 && lid >= 256;
     if (back) lid = total - 1 - (lid - 256);
     pslot = lid / nbh;
     bh = lid % nbh;
@@ -1262,8 +1262,12 @@ int launch_tile(KArgs a, hipStream_t st) {
   // Unpaired causal calls of more than one block per CU go heaviest block first over all heads: head after head put equal
   // (heavy) blocks on one CU (D = 128, causal; B=2 H=32 S=1000: 33.3 -> 28.0 us, B=2 H=32 S=2048: 98 -> 75 us, B=1 H=16
   // S=4096: 104 -> 86 us).  Pairs: from two rounds of the 512 resident workgroups, or where they are just one round.
-  a.lpt = (!BIAS && !a.cu_q && !a.pair && a.n_splits == 1 && a.is_causal &&
-           (int64_t)a.batch * a.heads_q * nblk > 256) ? 1 : 0;
+  // A grid of two blocks per CU runs its second half backwards at head_dim 65 ... 128, where just two workgroups are
+  // resident (B=1 H=16 S=4096: 87 against 88 us).  At head_dim 256 there is one per CU and the second half is a second
+  // round, whose heavy blocks must not come last (B=1 H=16 S=4096: 203 us backwards, 163 forwards, head after head 168;
+  // B=4 H=8 S=2048: 112, 91, 130); at head_dim 64 there are three (B=1 H=16 S=4096: 60.7 backwards, 58.6 forwards).
+  const int64_t blocks = (int64_t)a.batch * a.heads_q * nblk;
+  a.lpt = (!BIAS && !a.cu_q && !a.pair && a.n_splits == 1 && a.is_causal && blocks > 256) ? (DP == 128 && blocks <= 512 ? 2 : 1) : 0;
   a.hgroup = 1;
   if (BIAS && !a.cu_q && a.bias_sh == 0)
     for (int gsz = FA_HGROUP; gsz > 1; gsz >>= 1)
