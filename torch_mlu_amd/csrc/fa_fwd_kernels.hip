@@ -1259,15 +1259,29 @@ int launch_tile(KArgs a, hipStream_t st) {
   // packed: the kernel finds the pairs itself with one lane per sequence, in a loop over the block index
   if (a.cu_q && (a.batch > 64 || nblk > 1024)) a.pair = 0;
   a.n_mblk = (a.pair && !a.cu_q) ? (nblk + 1) / 2 : nblk;
-  // Unpaired causal calls of more than one block per CU go heaviest block first over all heads: head after head put equal
-  // (heavy) blocks on one CU (D = 128, causal; B=2 H=32 S=1000: 33.3 -> 28.0 us, B=2 H=32 S=2048: 98 -> 75 us, B=1 H=16
-  // S=4096: 104 -> 86 us).  Pairs: from two rounds of the 512 resident workgroups, or where they are just one round.
-  // A grid of two blocks per CU runs its second half backwards at head_dim 65 ... 128, where just two workgroups are
-  // resident (B=1 H=16 S=4096: 87 against 88 us).  At head_dim 256 there is one per CU and the second half is a second
-  // round, whose heavy blocks must not come last (B=1 H=16 S=4096: 203 us backwards, 163 forwards, head after head 168;
-  // B=4 H=8 S=2048: 112, 91, 130); at head_dim 64 there are three (B=1 H=16 S=4096: 60.7 backwards, 58.6 forwards).
-  const int64_t blocks = (int64_t)a.batch * a.heads_q * nblk;
-  a.lpt = (!BIAS && !a.cu_q && !a.pair && a.n_splits == 1 && a.is_causal && blocks > 256) ? (DP == 128 && blocks <= 512 ? 2 : 1) : 0;
+  // Unpaired causal calls of more than one block per CU: heaviest block first over all heads, or head after head.  The
+  // latter keeps a head's K and V in its XCD's L2, but with a multiple of 4 blocks per head it puts equal (heavy) blocks on
+  // the same CUs.  Heaviest first reads K and V from the last-level cache once more heads are under way than fit the L2s
+  // (many heads of short sequences; less of a loss where a tile takes longer: head_dim 64, dropout), and with a multiple of
+  // 4 blocks pays all the same as long as K and V fit that cache, or are read only 4 times.  Whole op, bf16, causal, us, head
+  // after head / heaviest first: head_dim 128, B=2 H=32 S=1000 33.3 / 28.0, S=2048 98 / 75, B=1 H=16 S=4096 104 / 86, B=10
+  // H=32 S=500 47 / 45, S=640 57 / 63 (dropout 77 / 75), B=30 H=32 S=130 36 / 42; head_dim 64, B=10 H=32 S=640 36 / 33.5,
+  // B=20 H=32 S=192 17.0 / 18.9; head_dim 256, B=5 H=32 S=640 79 / 78, B=10 H=32 S=256 54 / 49, S=500 135 / 110, S=384
+  // 72 / 78, S=900 334 / 310, B=30 H=32 S=640 416 / 527, B=16 H=32 S=900 522 / 563.
+  // Pairs: from two rounds of the 512 resident workgroups, or where they are just one round.
+  const int64_t heads = (int64_t)a.batch * a.heads_q, blocks = heads * nblk;
+  const int64_t kv_bytes = (int64_t)a.batch * a.heads_k * a.seqlen_k * DP * 4;
+  constexpr int kMostHeads = DP == 64 ? (DROP ? 2048 : 512) : (DP == 128 && DROP ? 384 : 192);
+  const bool spread = heads <= kMostHeads || nblk == 4 || (nblk % 4 == 0 && kv_bytes <= (384LL << 20)) ||
+                      ((DP == 256 || DROP) && nblk == 2 && a.seqlen_q > 224);
+  a.lpt = (!BIAS && !a.cu_q && !a.pair && a.n_splits == 1 && a.is_causal && blocks > 256 && spread) ? 1 : 0;
+  // A grid of two blocks per CU runs its second half backwards where just two workgroups are resident: head_dim 65 ... 128
+  // (B=1 H=16 S=4096: 87 against 88 us; with 2 or 3 blocks per head there is nothing to balance: B=5 H=32 S=300 16.4
+  // against 15.8), head_dim 64 with dropout (B=2 H=32 S=900: 21.3 against 22.5).  At head_dim 256 there is one per CU and
+  // the second half is a second round, whose heavy blocks must not come last (B=1 H=16 S=4096: 203 us backwards, 163
+  // forwards, head after head 168; B=4 H=8 S=2048: 112, 91, 130); at head_dim 64 without dropout there are three (B=1 H=16
+  // S=4096: 60.7 backwards, 58.6 forwards).
+  if (a.lpt && blocks <= 512 && ((DP == 128 && nblk >= 4) || (DP == 64 && DROP))) a.lpt = 2;
   a.hgroup = 1;
   if (BIAS && !a.cu_q && a.bias_sh == 0)
     for (int gsz = FA_HGROUP; gsz > 1; gsz >>= 1)
