@@ -40,6 +40,8 @@ def _check(q, k, v, causal, **kw):
     (1, 65, 1000),   # 520: more than two per CU
     (2, 62, 1000),   # 992 blocks = 496 pairs: one pair per resident workgroup
     (1, 520, 130),   # 1040 blocks, two per head
+    (8, 32, 300),    # 512 pairs, three blocks per head: paired at head_dim 128, heaviest first at 64, head after head at 256
+    (10, 32, 500),   # 1280 blocks, four per head
 ])
 @pytest.mark.parametrize("D", [64, 128, 256])
 def test_every_causal_block_is_computed(D, B, H, S):

@@ -1255,7 +1255,16 @@ int launch_tile(KArgs a, hipStream_t st) {
   if (!ensure_dynamic_lds<kfn>(lds)) return FA_ERR_LAUNCH;
   const int nblk = (a.seqlen_q + 127) / 128;
   const int64_t pairs = (int64_t)a.batch * a.heads_q * ((nblk + 1) / 2);
-  a.pair = (DP != 256 && a.n_splits == 1 && a.is_causal && nblk >= 2 && (pairs >= 1024 || (pairs > 480 && pairs <= 512))) ? 1 : 0;
+  // Pairs: from two rounds of the 512 resident workgroups on, or where they are just one round.  The latter only for one
+  // length (packed lengths differ and leave slots of the round empty: 8 sequences of 256 ... 1024 rows, 16 heads, head_dim 64
+  // 23 us unpaired against 26, head_dim 128 34 against 36, dropout 37 against 43; the price is equal lengths packed: 4 x 1000,
+  // 32 heads, head_dim 128 49 against 45), and where heaviest block first, below, is not the better order: head_dim 128 (B=4
+  // H=32 S=1000: paired 46 us, heaviest first 50; head_dim 64: 32 and 29.5, S=300 16.4 and 13), two blocks per head, and calls
+  // with a bias (B=4 H=32 S=1000, a bias per head, head_dim 128: paired 66 us, head after head 84; head_dim 64: 43, 57), of
+  // which not two blocks per head at head_dim 128 (B=16 H=32 S=248: 34.7 against 32.7; with dropout 36.7 against 40.3).
+  const bool one_round = pairs > 480 && pairs <= 512 && (!a.cu_q || a.batch == 1) &&
+                         (BIAS ? DROP || DP == 64 || nblk != 2 : DP == 128 || nblk == 2);
+  a.pair = (DP != 256 && a.n_splits == 1 && a.is_causal && nblk >= 2 && (pairs >= 1024 || one_round)) ? 1 : 0;
   // packed: the kernel finds the pairs itself with one lane per sequence, in a loop over the block index
   if (a.cu_q && (a.batch > 64 || nblk > 1024)) a.pair = 0;
   a.n_mblk = (a.pair && !a.cu_q) ? (nblk + 1) / 2 : nblk;
@@ -1268,7 +1277,6 @@ int launch_tile(KArgs a, hipStream_t st) {
   // H=32 S=500 47 / 45, S=640 57 / 63 (dropout 77 / 75), B=30 H=32 S=130 36 / 42; head_dim 64, B=10 H=32 S=640 36 / 33.5,
   // B=20 H=32 S=192 17.0 / 18.9; head_dim 256, B=5 H=32 S=640 79 / 78, B=10 H=32 S=256 54 / 49, S=500 135 / 110, S=384
   // 72 / 78, S=900 334 / 310, B=30 H=32 S=640 416 / 527, B=16 H=32 S=900 522 / 563.
-  // Pairs: from two rounds of the 512 resident workgroups, or where they are just one round.
   const int64_t heads = (int64_t)a.batch * a.heads_q, blocks = heads * nblk;
   const int64_t kv_bytes = (int64_t)a.batch * a.heads_k * a.seqlen_k * DP * 4;
   constexpr int kMostHeads = DP == 64 ? (DROP ? 2048 : 512) : (DP == 128 && DROP ? 384 : 192);
