@@ -164,6 +164,20 @@ def test_plan_split_count(batch, heads_k, seqlen_k, want):
     assert _plan(p) == (capi.FA_OK, capi.FA_KERNEL_SPLITKV, want)
 
 
+@pytest.mark.parametrize("batch,head_dim,seqlen_k,want", [
+    (1, 128, 512, 1), (8, 128, 512, 1), (20, 64, 512, 1), (64, 96, 512, 1),   # short caches: whole, whatever the batch ...
+    (2, 256, 512, 4), (8, 256, 512, 4),                                       # ... but at head_dim 256
+    (16, 128, 1024, 4), (20, 128, 1024, 1), (20, 128, 2048, 1), (20, 256, 512, 1), (20, 256, 1024, 4), (24, 128, 1408, 1),
+    (62, 128, 2048, 1), (64, 128, 2048, 1), (64, 128, 8192, 2), (64, 256, 8192, 3),   # two whole rounds
+    (24, 128, 2048, 1), (33, 128, 2048, 3), (33, 256, 2048, 1), (33, 64, 2048, 1),    # one and a half to three rounds
+    (32, 128, 8192, 6), (33, 128, 8192, 6), (33, 64, 3072, 3), (256, 128, 8192, 1),
+    (1, 128, 32768, 64), (16, 128, 16384, 12),
+])
+def test_plan_split_count_of_ragged_lengths(batch, head_dim, seqlen_k, want):
+    p = _good(batch=batch, heads_q=32, heads_k=8, seqlen_q=1, seqlen_k=seqlen_k, head_dim=head_dim, is_causal=0, seqused_k=0x8000)
+    assert _plan(p) == (capi.FA_OK, capi.FA_KERNEL_SPLITKV, want)
+
+
 @pytest.mark.parametrize("over,kern,ns", [
     (dict(batch=4, heads_q=32, heads_k=32, seqlen_q=4096, seqlen_k=4096), "tile", 1),     # the headline prefill
     (dict(batch=1, heads_q=32, heads_k=8, seqlen_q=128, seqlen_k=32768), "tile", 16),     # a chunk against a cache

@@ -117,23 +117,30 @@ def test_decode_slices_around_the_blocks_of_a_wavefront(D, used):
         assert (lse - want_l).abs().max().item() <= LSE_TOL
 
 
-
 @pytest.mark.parametrize("D", [64, 128, 256])
-@pytest.mark.parametrize("B", [47, 48, 64, 65])   # 188 units: sliced; 192, 256: whole, one per CU; 260: whole, two per CU
-def test_ragged_paged_units_around_one_per_cu(D, B):
-    Hq, Hk, page, per = 8, 4, 32, 10
+@pytest.mark.parametrize("B,per,ns", [
+    (47, 10, 0), (48, 10, 0), (64, 10, 0), (65, 10, 0),   # 188 ... 260 units of up to 320 keys: whole (sliced at head_dim 256)
+    (80, 40, 0),    # 320 of 1280: whole, four wavefronts
+    (66, 64, 0),    # 264 of 2048: three slices at head_dim 128
+    (126, 40, 0),   # 504 of 1280: two rounds, whole
+    (124, 81, 0),   # 496 of 2592: two rounds, two slices
+    (5, 50, 0),     # 20 of 1600: twelve slices
+    (5, 200, 2),    # 20 of 6400: two long slices, four wavefronts
+])
+def test_ragged_paged_units_around_one_per_cu(D, B, per, ns):
+    Hq, Hk, page = 8, 4, 32
     q = _randn((B, Hq, 1, D), 11, HF)
     kp, vp = _randn((B * per, page, Hk, D), 12, HF), _randn((B * per, page, Hk, D), 13, HF)
     g = torch.Generator(device=DEV).manual_seed(14)
     table = torch.randperm(B * per, generator=g, device=DEV).to(torch.int32).reshape(B, per)
     lens = torch.randint(1, per * page + 1, (B,), generator=g, device=DEV).to(torch.int32)
     lens[0], lens[-1] = per * page, 1
-    out, lse = capi.fa_forward_paged(q, kp, vp, table, lens)
-    k, v = (t[table.long()].reshape(B, per * page, Hk, D).transpose(1, 2).repeat_interleave(Hq // Hk, 1).float() for t in (kp, vp))
-    s = (q.float() * k).sum(-1) / math.sqrt(D)   # [B, Hq, keys]
+    out, lse = capi.fa_forward_paged(q, kp, vp, table, lens, num_splits=ns)
+    k, v = (t[table.long()].reshape(B, per * page, Hk, D).transpose(1, 2).float() for t in (kp, vp))
+    s = (q.float().reshape(B, Hk, -1, D) @ k.transpose(2, 3).contiguous()).reshape(B, Hq, -1) / math.sqrt(D)   # [B, Hq, keys]
     s.masked_fill_(torch.arange(per * page, device=DEV)[None, None, :] >= lens[:, None, None], float("-inf"))
     want_l = torch.logsumexp(s, -1)
-    want = (torch.exp(s - want_l[..., None])[..., None] * v).sum(2)
+    want = (torch.exp(s - want_l[..., None]).reshape(B, Hk, -1, per * page) @ v).reshape(B, Hq, D)
     assert (out[:, :, 0].float() - want).abs().max().item() <= OUT_TOL[HF]
     assert (lse[:, :, 0] - want_l).abs().max().item() <= LSE_TOL
 

@@ -1318,17 +1318,15 @@ int launch_splitkv(const KArgs& a, hipStream_t st) {
   return a.n_splits > 1 ? launch_merge<T>(a, st) : FA_OK;
 }
 
-// Sequences of one length: four wavefronts and most of a CU's LDS per workgroup, whose slices are equal and in step
-// (6.0 TB/s at B = 64, 8192 keys; two wavefronts: 5.6).  Ragged lengths: half the size, so that two workgroups share a CU
-// and one's start and merge are covered by the other's loads (512 units of up to 512 keys: 21 against 24 us), except where
-// there is one workgroup per CU at most, which then needs all of the CU's loads in flight (212 units of up to 1728 keys: 29
-// against 35 us).
+// Sequences of one length: four wavefronts and, at head_dim 128, most of a CU's LDS per workgroup, whose slices are equal and
+// in step (6.0 TB/s at B = 64, 8192 keys; two wavefronts: 5.6).  Ragged lengths: see ragged_half().
 template <typename T, bool DROP>
 int dispatch_splitkv(const KArgs& a, int dp, hipStream_t st) {
-  const bool ragged = (a.seqused_k || a.cu_q) && (a.n_splits > 1 || (int64_t)a.batch * a.heads_k > 256);
-  if (dp == 64) return ragged ? launch_splitkv<T, 64, 2, DROP>(a, st) : launch_splitkv<T, 64, 4, DROP>(a, st);
-  if (dp == 128) return ragged ? launch_splitkv<T, 128, 2, DROP>(a, st) : launch_splitkv<T, 128, 4, DROP>(a, st);
-  return launch_splitkv<T, 256, 2, DROP>(a, st);
+  if (dp == 64) return launch_splitkv<T, 64, 4, DROP>(a, st);
+  if (dp == 256) return launch_splitkv<T, 256, 2, DROP>(a, st);
+  if ((a.seqused_k || a.cu_q) && ragged_half(dp, (int64_t)a.batch * a.heads_k, a.seqlen_k, a.n_splits))
+    return launch_splitkv<T, 128, 2, DROP>(a, st);
+  return launch_splitkv<T, 128, 4, DROP>(a, st);
 }
 
 template <typename T>

@@ -97,6 +97,56 @@ inline int validate(const fa_fwd_params* p) {
   return FA_OK;
 }
 
+// Split-KV kernel, ragged lengths (known on the device only; `rows`, the longest possible one, is what the host sees; a
+// sequence's slices are cut from its own length; units = sequences x kv heads).  More slices even out the lengths over the
+// CUs and cost a start, partials and a merge launch; a full batch has nothing to even out.  Measured with every sequence
+// full, with lengths of 1/4 ... 1 and 1/16 ... 1 of the longest, and with one long sequence among short ones, 8 ... 1024
+// units of 512 ... 32768 keys (us, whole op; head_dim 128 where not said):
+//   - short caches stay whole: below 768 rows a slice saves less than it costs (160 units of 512 keys: one slice 11, four
+//     17), from 144 units, more than half the CUs, below 2560 (160 of 1024 18 and 24, of 2048 30 and 37; lengths 1/4 ... 1 25
+//     and 27), from 192 below 1536.  At head_dim 256, with twice the bytes a row, slices pay below 144 units (16 of 512: 12
+//     against 19) and from 768 rows on (160 of 512: 26 and 32);
+//   - two whole rounds of the CUs: two slices at most (512 units of 8192 keys: full 361 in two, 382 in three; lengths 1/4 ...
+//     1: 262 and 265);
+//   - otherwise up to three rounds of the 512 resident half-size workgroups while slices keep 512 rows, 640 from 192 units
+//     on (1024 at head_dim 64: 448 of 2048 whole 31, in three 33), where it takes two rounds to be worth it, or one and a
+//     half beyond 256 units (212 of 1728: whole 29, in three 36; 264 of 2048: 60 and 50); at least one round while slices
+//     keep 128.
+// What a full batch pays for that, against long slices or none: 128 units of 16384 keys 200 for 194 (lengths 1/4 ... 1: 122
+// for 154), 224 of 8192 176 for 168 (125 for 146), 256 of 8192 199 for 192 (131 for 150).
+inline bool two_rounds(int dp, int64_t units) { return dp == 128 && units >= 496 && units <= 512; }
+inline int ragged_slices(int dp, int64_t units, int64_t rows) {
+  const int64_t whole_below = units < 144 ? (dp == 256 ? 0 : 768) : (dp == 256 ? 768 : (units < 192 ? 2560 : 1536));
+  if (rows < whole_below) return 1;
+  if (two_rounds(dp, units)) return rows >= 2560 ? 2 : 1;
+  auto most = [&](int64_t wgs, int64_t least) {  // slices that make `wgs` workgroups and keep `least` rows
+    const int64_t fill = (wgs + units - 1) / units, cap = rows / least;
+    return fill < cap ? fill : cap;
+  };
+  int64_t n;
+  if (units < 192) {
+    const int64_t one = most(512, 128), three = most(1536, 512);
+    n = one > three ? one : three;
+  } else {
+    n = most(1536, dp == 64 ? 1024 : 640);
+    if (units * n < (dp == 256 || units <= 256 || n < 3 ? 1024 : 768) || (dp == 64 && n < 3)) n = 1;
+  }
+  if (n > 8) n &= ~(int64_t)3;
+  return (int)(n < 1 ? 1 : (n > FA_MAX_SPLITS ? FA_MAX_SPLITS : n));
+}
+// Two wavefronts a workgroup instead of four?  At head_dim 128 a workgroup of four has its CU to itself; of two, two share
+// one, and one's start and merge are covered by the other's loads.  Four where a workgroup streams for long, is alone on its
+// CU or in step with the others, and for few rows in something over one round (us: 512 units of 512 keys, full: four 27, two
+// 25; 512 of 1024 43 and 46; 264 of 1024 35 and 32; 448 of 1024 39 and 41; 264 of 16384 in six slices 383 and 394, lengths
+// 1/4 ... 1 235 and 250; 512 of 8192 in two slices 361 and 379).  At head_dim 64 two workgroups of four share a CU anyway
+// (512 of 8192 in three slices, lengths 1/4 ... 1: four 138, two 146); at head_dim 256 there are no other than of two.
+inline bool ragged_half(int dp, int64_t units, int64_t rows, int slices) {
+  if (dp != 128) return false;
+  if (two_rounds(dp, units)) return rows < 1024;
+  if (slices > 1) return rows < (int64_t)2560 * slices;
+  return units > 256 && !(units >= 320 && units <= 768 && rows >= 1024 && rows < 1536);
+}
+
 inline void plan(const fa_fwd_params* p, int* kernel, int* splits) {
   int kern = p->kernel;
   const int group = p->heads_q / p->heads_k;
@@ -120,21 +170,7 @@ inline void plan(const fa_fwd_params* p, int* kernel, int* splits) {
       const int64_t units = (int64_t)p->batch * p->heads_k;
       ns = 1;
       if (p->seqused_k || p->cu_seqlens_q) {
-        // Ragged lengths, known on the device only: seqlen_k is the longest possible one, and a sequence's slices are
-        // cut from its own length.  One round of the 512 resident (half-size) workgroups is wanted while slices of the
-        // longest keep 128 rows, and up to three, to even out what the dispatcher hands the CUs, while they keep 512.
-        // Where the units alone come near one per CU, slices and their merge have to buy more: two whole rounds of 640
-        // rows, or none.  Measured on 2 ... 64 paged sequences of up to 512 ... 16k keys: within 5 % of the best count
-        // (212 units of 1728 keys: one slice 29 us, three 36; 256 of 2048: 36, two 41; 256 of 4096: 63, six 61).
-        auto most = [&](int64_t wgs, int64_t rows) {
-          const int64_t fill = (wgs + units - 1) / units, cap = p->seqlen_k / rows;
-          return fill < cap ? fill : cap;
-        };
-        const int64_t one = most(512, 128), three = most(1536, units >= 192 ? 640 : 512);
-        int64_t n = one > three ? one : three;
-        if (units >= 192) n = units * three >= 1024 ? three : 1;
-        if (n > 8) n &= ~(int64_t)3;
-        ns = (int)(n < 1 ? 1 : (n > FA_MAX_SPLITS ? FA_MAX_SPLITS : n));
+        ns = ragged_slices(padded_dim(p->head_dim), units, p->seqlen_k);
       } else {
         while (ns * 2 <= FA_MAX_SPLITS && units * ns * 2 <= kCUs) ns *= 2;
         while (ns > 1 && p->seqlen_k / ns < 2048 && units * (ns / 2) >= kCUs / 2) ns /= 2;
