@@ -44,7 +44,52 @@ static long push_fwd(const fa_fwd_params& p) {
   return n + 1000003;
 }
 
+// key_block_tiles_before() against a sum over the blocks as the dK/dV kernel counts them, and the slots that bwd_slices()
+// plans from it: those of a block's slices end before the next block's begin, and inside what the workspace holds.
+static long check_key_block_slots() {
+  long bad = 0;
+  for (int causal : {0, 1})
+    for (int nq = 0; nq <= 9; ++nq)
+      for (int off = -1500; off <= 1500; off += (off % 64 == 0 ? 1 : (off % 64 == 1 || off % 64 == -63 ? 61 : 1))) {
+        int64_t sum = 0;
+        for (int p = 0; p <= 12; ++p) {
+          if (key_block_tiles_before(p, nq, off, causal != 0) != sum) ++bad;
+          const int begin = causal ? (128 * p - off > 0 ? (128 * p - off) / 64 : 0) : 0;
+          sum += nq - begin > 0 ? nq - begin : 0;
+        }
+      }
+  for (int group : {1, 4, 7, 16})
+    for (int sq : {1, 64, 130, 300, 500, 1024, 1900, 4096})
+      for (int sk : {1, 64, 129, 500, 1500, 4096})
+        for (int d : {64, 128, 256})
+          for (int mask : {0, 1, 2}) {
+            fa_bwd_params p;
+            memset(&p, 0, sizeof(p));
+            p.batch = 2; p.heads_q = 2 * group; p.heads_k = 2; p.seqlen_q = sq; p.seqlen_k = sk; p.head_dim = d; p.is_causal = mask;
+            const BwdSlices r = bwd_slices(&p);
+            const double tensors = 8.0 * d * (2.0 * sq * p.heads_q + 2.0 * sk * p.heads_k);
+            if ((double)r.bytes > 1.25 * tensors) ++bad;
+            if (r.count == 1) {
+              bad += r.bytes != 0;
+              continue;
+            }
+            const int64_t nq = (sq + 63) / 64, nk = (sk + 127) / 128, off = mask == 2 ? 0 : sk - sq;
+            for (int64_t i = 0; i < nk; ++i) {
+              const int64_t s0 = group * key_block_tiles_before(i, nq, off, mask != 0);
+              const int64_t s1 = group * key_block_tiles_before(i + 1, nq, off, mask != 0);
+              const int64_t cuts = s1 == s0 ? 1 : (s1 - s0 + r.iters - 1) / r.iters;
+              if (cuts > r.count || s0 / r.iters + i + cuts > s1 / r.iters + i + 1 || s1 / r.iters + i + 1 > r.slots) ++bad;
+            }
+            if (r.bytes != (size_t)r.slots * 4 * 128 * padded_dim(d) * 4 * 2) ++bad;
+          }
+  return bad;
+}
+
 int main() {
+  if (const long bad = check_key_block_slots()) {
+    fprintf(stderr, "key block slots: %ld wrong\n", bad);
+    return 1;
+  }
   long sink = 0, count = 0;
   const int32_t big = 0x7fffffff;
   for (int B : {1, 2, 64, 4096, big})

@@ -239,18 +239,33 @@ def test_bwd_validate_accepts_good_params_and_sizes_delta_scratch():
     assert L.fa_bwd_validate(ctypes.byref(full)) == capi.FA_OK
 
 
-@pytest.mark.parametrize("Hq,Hk,S,D,slices", [
-    (28, 4, 4096, 128, 16),   # 448 steps, 112 a CU: slices of 28
-    (14, 2, 130, 128, 2),     # 21 steps: slices of 11
-    (16, 16, 2048, 128, 1),   # 32 steps, 16 a CU
-    (32, 32, 4096, 128, 1),
-    (16, 4, 2048, 64, 8),     # 128 steps, slices of 16
+@pytest.mark.parametrize("Hq,Hk,S,D,slots", [
+    (28, 4, 4096, 128, 4 * 263),   # 448 steps, 112 a CU; slices of 32
+    (14, 2, 130, 128, 2 * 4),      # 21 steps: slices of 11
+    (16, 16, 2048, 128, 0),        # 32 steps, 16 a CU
+    (32, 32, 4096, 128, 0),
+    (16, 4, 2048, 64, 4 * 84),     # 128 steps; slices of 16
+    (8, 8, 1024, 256, 0),
+    (8, 2, 300, 256, 2 * 6),       # 20 steps; slices of 10
 ])
-def test_bwd_workspace_holds_the_slices_partial_sums(Hq, Hk, S, D, slices):
+def test_bwd_workspace_holds_the_slices_partial_sums(Hq, Hk, S, D, slots):
+    """As many slots of 128 key rows (dK and dV, fp32) as slices can begin, and no more bytes than 5/4 of the call's tensors."""
     p = _good_bwd(batch=1, heads_q=Hq, heads_k=Hk, seqlen_q=S, seqlen_k=S, head_dim=D)
-    planes = 2 * (S * Hq * 4)
-    parts = 0 if slices == 1 else Hk * ((S + 127) // 128) * slices * 2 * (128 * D * 4)
+    planes, parts = 2 * (S * Hq * 4), slots * 2 * (128 * D * 4)
     assert capi.lib().fa_bwd_workspace_bytes(ctypes.byref(p)) == planes + parts
+    assert parts <= 5 * (Hq + Hk) * S * D * 2
+
+
+@pytest.mark.parametrize("batch,Hq,Hk,longest,total", [
+    (8, 16, 4, 1500, 7444), (8, 16, 4, 1500, 12000), (2, 28, 4, 4096, 4200), (32, 16, 2, 700, 9000), (1, 16, 2, 1500, 1500),
+    (64, 16, 1, 4096, 5000),
+])
+def test_bwd_workspace_of_packed_sequences_is_modest(batch, Hq, Hk, longest, total):
+    """Partial sums of packed sequences are sized by the rows there are, not by the longest times the batch."""
+    p = _good_bwd(batch=batch, heads_q=Hq, heads_k=Hk, seqlen_q=longest, seqlen_k=longest, head_dim=128, cu_seqlens_q=0xa000,
+                  cu_seqlens_k=0xb000, total_q=total)
+    need = capi.lib().fa_bwd_workspace_bytes(ctypes.byref(p))
+    assert need <= 2 * (total * Hq * 4 + 15) + 5 * (Hq + Hk) * total * 128 * 2
 
 
 @pytest.mark.parametrize("over,rc", [

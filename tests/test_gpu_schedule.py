@@ -210,3 +210,70 @@ def test_sliced_key_blocks_packed(Hq, Hk, D):
     for i, n in enumerate(lens):
         if n:
             _check_grads([row(t, i) for t in got], _grad_reference(*(row(t, i) for t in (q, k, v, do)), True), BF)
+
+
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("lens_q,lens_k", [
+    ([130] * 6, [1500] * 6),                                   # more key blocks than self-attention has: room for some sequences only
+    ([1, 200, 0, 64] * 20 + [900], [1, 200, 0, 64] * 20 + [900]),   # more sequences than lanes, empty ones among them
+])
+def test_sliced_key_blocks_packed_slots(lens_q, lens_k, causal):
+    Hq, Hk, D = 28, 2, 64
+    cq, ck = [0], [0]
+    for n, m in zip(lens_q, lens_k):
+        cq.append(cq[-1] + n)
+        ck.append(ck[-1] + m)
+    q, k, v, do = _randn((cq[-1], Hq, D), 44, BF), _randn((ck[-1], Hk, D), 45, BF), _randn((ck[-1], Hk, D), 46, BF), _randn((cq[-1], Hq, D), 47, BF)
+    cuq, cuk = (torch.tensor(c, dtype=torch.int32, device=DEV) for c in (cq, ck))
+    out, lse = capi.fa_forward_packed(q, k, v, cuq, cuk, max(lens_q), max(lens_k), is_causal=causal)
+    got = capi.fa_backward_packed(do, q, k, v, out, lse, cuq, cuk, max(lens_q), max(lens_k), is_causal=causal)
+    row = lambda t, c, i: t[c[i]:c[i + 1]].transpose(0, 1)[None]
+    for i in (0, 1, len(lens_q) // 2 + 1, len(lens_q) - 1):
+        want = _grad_reference(row(q, cq, i), row(k, ck, i), row(v, ck, i), row(do, cq, i), causal)
+        _check_grads([row(got[0], cq, i), row(got[1], ck, i), row(got[2], ck, i)], want, BF)
+
+
+def test_backward_without_room_for_partial_sums():
+    """Less workspace than asked for, but room for the two planes: whole key blocks."""
+    q, k, v, do = (_randn(s, 60 + i, BF) for i, s in enumerate([(1, 14, 300, 128), (1, 2, 500, 128), (1, 2, 500, 128), (1, 14, 300, 128)]))
+    out, lse = capi.fa_forward_dense(q, k, v, is_causal=True)
+    real = capi.lib()
+    planes = 2 * 14 * 300 * 4
+
+    class Short:
+        def __init__(self, size):
+            self.fa_bwd_workspace_bytes = lambda p: size
+
+        def __getattr__(self, name):
+            return getattr(real, name)
+
+    try:
+        assert capi.lib() is real
+        capi._lib = Short(planes)
+        _check_grads(capi.fa_backward_dense(do, q, k, v, out, lse, is_causal=True), _grad_reference(q, k, v, do, True), BF)
+        capi._lib = Short(planes - 16)
+        with pytest.raises(capi.FaFwdError):
+            capi.fa_backward_dense(do, q, k, v, out, lse, is_causal=True)
+    finally:
+        capi._lib = real
+
+
+def test_training_step_close_to_the_memory_limit():
+    """The op falls back to whole key blocks where the partial sums of sliced ones do not fit."""
+    import torch.nn.functional as F
+
+    q, k, v = (_randn(s, 70 + i, BF).requires_grad_() for i, s in enumerate([(1, 28, 2048, 128), (1, 4, 2048, 128), (1, 4, 2048, 128)]))
+    do = _randn((1, 28, 2048, 128), 73, BF)
+    step = lambda: torch.autograd.grad(F.scaled_dot_product_attention(q, k, v, is_causal=True, enable_gqa=True), (q, k, v), do)
+    want = step()
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    total = torch.cuda.get_device_properties(0).total_memory
+    try:   # room for the output, the gradients and the planes (36 MiB), not for 60 MiB of partial sums
+        torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (60 << 20)) / total)
+        got = step()
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    for a, b in zip(got, want):
+        assert torch.isfinite(a).all() and (a.float() - b.float()).abs().max().item() <= 2 * 2.0 ** -8 * max(b.abs().max().item(), 0.25)
+    assert torch.equal(got[0], want[0]) and not torch.equal(got[1], want[1])   # dQ as before; dK summed in another order

@@ -41,6 +41,7 @@
 
 #include "fa_bwd.h"
 #include "fa_fwd.h"
+#include "fa_host.h"
 
 namespace torch_mlu_amd {
 
@@ -384,6 +385,19 @@ scaled_dot_product_flash_attention(const at::Tensor& query, const at::Tensor& ke
                          philox_offset, debug_attn_mask);
 }
 
+// Scratch of a backward call.  What does not fit into memory any more with the partial sums of sliced key blocks still runs
+// without them, as slow as whole blocks are.
+at::Tensor backward_workspace(const fa_bwd_params& p, const at::TensorOptions& bytes) {
+  const size_t need = fa_bwd_workspace_bytes(&p), least = 2 * fa::host::bwd_ws_plane(&p);
+  auto make = [&](size_t n) { return at::empty({static_cast<int64_t>(n > 0 ? n : 16)}, bytes); };
+  if (need == least) return make(need);
+  try {
+    return make(need);
+  } catch (const c10::OutOfMemoryError&) {
+    return make(least);
+  }
+}
+
 // ---- _flash_attention_backward --------------------------------------------------------------------------------
 // cnnl__flash_attention_backward, attention.cpp:305-348, and the checks of mha_varlen_bwd
 // (FlashAttention_internal.cpp:288-366).  3-D inputs: packed [T, H, D] with cum_seq (the reference's only mode);
@@ -476,10 +490,9 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor> flash_attention_backward(
     dq.zero_(); dk.zero_(); dv.zero_();
     return std::make_tuple(dq, dk, dv);
   }
-  const size_t ws_bytes = fa_bwd_workspace_bytes(&p);
-  at::Tensor ws = at::empty({static_cast<int64_t>(ws_bytes > 0 ? ws_bytes : 16)}, q.options().dtype(at::kByte));
+  const at::Tensor ws = backward_workspace(p, q.options().dtype(at::kByte));
   hipStream_t stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(q.device().index()).stream();
-  const int rc = fa_bwd_launch(&p, ws.data_ptr(), ws_bytes, stream);
+  const int rc = fa_bwd_launch(&p, ws.data_ptr(), static_cast<size_t>(ws.numel()), stream);
   TORCH_CHECK(rc == FA_OK, "fa_bwd_launch failed: ", fa_fwd_error_string(rc), " (rc=", rc, ")");
   g_launches.fetch_add(1, std::memory_order_relaxed);
   return std::make_tuple(dq, dk, dv);
@@ -898,10 +911,9 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor, at::Tensor> efficient_attention_b
     dq.zero_(); dk.zero_(); dv.zero_();
     if (want_dbias) dbias.zero_();
   } else {
-    const size_t ws_bytes = fa_bwd_workspace_bytes(&p);
-    at::Tensor ws = at::empty({static_cast<int64_t>(ws_bytes > 0 ? ws_bytes : 16)}, q.options().dtype(at::kByte));
+    const at::Tensor ws = backward_workspace(p, q.options().dtype(at::kByte));
     hipStream_t stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(q.device().index()).stream();
-    const int rc = fa_bwd_launch(&p, ws.data_ptr(), ws_bytes, stream);
+    const int rc = fa_bwd_launch(&p, ws.data_ptr(), static_cast<size_t>(ws.numel()), stream);
     TORCH_CHECK(rc == FA_OK, "fa_bwd_launch failed: ", fa_fwd_error_string(rc), " (rc=", rc, ")");
     g_launches.fetch_add(1, std::memory_order_relaxed);
   }

@@ -100,11 +100,45 @@ struct BArgs {
   float* part;
   int64_t part_dv;            // floats from the partials of dK to those of dV
   int32_t n_slices, slice_iters;
+  int32_t part_slots;         // slots of 128 key rows: of each (sequence, kv head); packed: of each kv head
 };
 
 // slices of a key block with `niter` steps: as even as possible, none longer than slice_iters
 __device__ __forceinline__ int dkv_slices(const BArgs& a, int niter) {
   return min(a.n_slices, max(1, (niter + a.slice_iters - 1) / a.slice_iters));
+}
+
+// Slot of the first slice of key block `pslot` of sequence b (Lq rows, Lk keys), kv head hk, among the partial sums; -1: there
+// is no room for this sequence, its blocks stay whole (packed only, where the host knows the total length but not the
+// sequences').  Every lane of the wavefront calls it.  The dense products fit 31 bits (bwd_slices); a packed sequence whose
+// products do not is one there is no room for.
+__device__ __forceinline__ int dkv_first_slot(const BArgs& a, int b, int hk, int pslot, int Lq, int Lk) {
+  auto before = [&](int64_t p, int lq, int lk) -> int64_t {  // steps of the first p key blocks of a sequence
+    return fa::host::key_block_tiles_before(p, (lq + 63) / 64, a.causal_tl ? 0 : lk - lq, a.is_causal != 0) * a.group;
+  };
+  const unsigned iters = (unsigned)a.slice_iters;
+  const int mine = (int)((unsigned)before(pslot, Lq, Lk) / iters) + pslot;
+  if (!a.cu_q) return (b * a.heads_k + hk) * a.part_slots + mine;
+  // slots of each sequence up to this one, a lane each; sums are cut off where they exceed what there is
+  const int lane = threadIdx.x & 63, cap = a.part_slots + 1;
+  int base = 0, own = 0;
+  for (int s0 = 0; s0 <= b; s0 += 64) {
+    const int s = s0 + lane;
+    int slots = 0;
+    if (s <= b) {
+      const int lq = max(a.cu_q[s + 1] - a.cu_q[s], 0), lk = max(a.cu_k[s + 1] - a.cu_k[s], 0);
+      const int nk = (lk + 127) / 128;
+      const int64_t steps = before(nk, lq, lk);
+      slots = steps > 0x7fffffff ? cap : (int)min((unsigned)steps / iters + (unsigned)nk, (unsigned)cap);
+    }
+    if (b - s0 < 64) own = __builtin_amdgcn_readlane(slots, __builtin_amdgcn_readfirstlane(b - s0));
+    if (s >= b) slots = 0;
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) slots += __shfl_xor(slots, o);
+    base = min(base + __builtin_amdgcn_readfirstlane(slots), cap);
+  }
+  if (base + own > a.part_slots) return -1;
+  return base * a.heads_k + hk * own + mine;
 }
 
 // One swizzle for tiles that are read both by rows (16 lanes = 16 consecutive rows, same logical chunk) and
@@ -687,13 +721,11 @@ __device__ __forceinline__ void dkv_block(const BArgs& a, unsigned char* smem, i
   const int jq_end = (Lq + BQ - 1) / BQ;
   const int nq = max(0, jq_end - jq_begin);
   // flattened (query head of the group, query tile); a slice takes steps it0 ... it1 - 1
-  int it0 = 0, it1 = nq * a.group, ns = 1;
+  const int niter = nq * a.group;
+  int it0 = 0, it1 = niter, ns = 1;
   if (a.n_slices > 1) {
-    ns = dkv_slices(a, it1);
+    ns = dkv_slices(a, niter);
     if (slice >= ns) return;
-    const int64_t n = it1;
-    it0 = (int)(n * slice / ns);
-    it1 = (int)(n * (slice + 1) / ns);
   }
 
   // ---- K and V fragments of my key row (B operands) ----
@@ -712,6 +744,19 @@ __device__ __forceinline__ void dkv_block(const BArgs& a, unsigned char* smem, i
       }
       kf[ks] = __builtin_bit_cast(s16x8, x);
       vf[ks] = __builtin_bit_cast(s16x8, y);
+    }
+  }
+
+  int slot = 0;
+  if (ns > 1) {  // (behind the loads above, which cover the look at the other sequences' lengths)
+    slot = dkv_first_slot(a, b, hk, pslot, Lq, Lk);
+    if (slot < 0) {
+      if (slice > 0) return;
+      ns = 1;
+    } else {
+      slot += slice;
+      it0 = (int)((int64_t)niter * slice / ns);
+      it1 = (int)((int64_t)niter * (slice + 1) / ns);
     }
   }
 
@@ -1086,7 +1131,7 @@ __device__ __forceinline__ void dkv_block(const BArgs& a, unsigned char* smem, i
 
   if (ns > 1) {
     // a slice's sums stay as the MFMAs left them: 16 bytes per lane, 1 KiB per store instruction
-    const int64_t at = ((((int64_t)pslot * (a.batch * a.heads_k) + bhk) * a.n_slices + slice) * 4 + wave) * (32 * DP) + lane * 4;
+    const int64_t at = ((int64_t)slot * 4 + wave) * (32 * DP) + lane * 4;
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
@@ -1200,7 +1245,9 @@ __global__ void __launch_bounds__(256) fa_bwd_dkv_merge_kernel(const BArgs a) {
   const int jq_begin = a.is_causal ? max(0, n0 - off) / BQ : 0;
   const int ns = dkv_slices(a, max(0, (Lq + BQ - 1) / BQ - jq_begin) * a.group);
   if (ns == 1) return;  // written by the dK/dV kernel
-  const float* src = a.part + (is_dv ? a.part_dv : 0) + ((int64_t)unit * a.n_slices * 4 + part) * (32 * DP) + tid * 4;
+  const int slot = dkv_first_slot(a, b, hk, pslot, Lq, Lk);
+  if (slot < 0) return;
+  const float* src = a.part + (is_dv ? a.part_dv : 0) + ((int64_t)slot * 4 + part) * (32 * DP) + tid * 4;
   f32x4 sum[MB];
 #pragma unroll
   for (int i = 0; i < MB; ++i) sum[i] = *(const f32x4*)(src + i * 1024);
@@ -1307,16 +1354,17 @@ size_t fa_bwd_workspace_bytes(const fa_bwd_params* p) {
 int fa_bwd_launch(const fa_bwd_params* p, void* workspace, size_t workspace_bytes, void* stream) {
   const int rc = bwd_validate(p);
   if (rc != FA_OK) return rc;
-  const size_t need = bwd_ws_bytes(p);
-  if (need > 0 && (!workspace || workspace_bytes < need || ((uintptr_t)workspace & 15))) return FA_ERR_BAD_ARG;
+  const size_t need = bwd_ws_bytes(p), least = 2 * bwd_ws_plane(p);
+  if (least > 0 && (!workspace || workspace_bytes < least || ((uintptr_t)workspace & 15))) return FA_ERR_BAD_ARG;
   BArgs a;
   a.q = (const unsigned char*)p->q; a.k = (const unsigned char*)p->k; a.v = (const unsigned char*)p->v;
   a.o = (const unsigned char*)p->out; a.dout = (const unsigned char*)p->dout; a.lse = p->lse;
   a.dq = (unsigned char*)p->dq; a.dk = (unsigned char*)p->dk; a.dv = (unsigned char*)p->dv;
   a.delta = (float*)workspace;
   a.lse2 = (float*)((unsigned char*)workspace + bwd_ws_plane(p));
-  const host::BwdSlices sl = host::bwd_slices(p);
-  a.n_slices = sl.count; a.slice_iters = sl.iters;
+  host::BwdSlices sl = host::bwd_slices(p);
+  if (workspace_bytes < need) sl.count = 1;  // no room for partial sums: whole key blocks
+  a.n_slices = sl.count; a.slice_iters = sl.iters; a.part_slots = sl.slots;
   a.part = (float*)((unsigned char*)workspace + 2 * bwd_ws_plane(p));
   a.part_dv = (int64_t)(sl.bytes / 8);
   a.cu_q = p->cu_seqlens_q; a.cu_k = p->cu_seqlens_k;

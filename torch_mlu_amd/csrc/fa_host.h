@@ -286,39 +286,81 @@ inline size_t bwd_ws_plane(const fa_bwd_params* p) {
 // rows 882 -> 575, 700 rows 145 -> 60; 32 / 8, 2048 rows 272 -> 195, 4096 rows 642 -> 607; batch 4, 16 / 4, head_dim 64,
 // 2048 rows 225 -> 165; 8 packed sequences of 187 ... 1500 rows, 16 / 4, 250 -> 232.  On the other side of the line:
 // 16 / 16, 2048 rows 113 -> 133; 8 / 8, 4096 rows 209 -> 222; batch 2, 16 / 8, head_dim 256, 2000 rows 331 -> 423.
+//
+// The partial sums take at most 5/4 of the memory of the call's own tensors (q, out, dout, dq and k, v, dk, dv): slices get
+// longer until they do, or the blocks stay whole.
+//
+// Pairs of (128-key block, 64-row query tile that sees some of its keys) in the first p key blocks: off = Lk - Lq, or 0 for
+// the top-left mask.  Block i sees the tiles from max(0, 128 i - off) / 64 = max(0, 2 i + t) on.  (constexpr: the kernels
+// call it too)
+constexpr int64_t key_block_tiles_before(int64_t p, int64_t nq, int64_t off, bool causal) {
+  if (!causal) return p * nq;
+  const int64_t t = (-off) >> 6;
+  const int64_t all = t > 0 ? 0 : -t / 2 + 1;         // blocks that see every tile
+  const int64_t some = (nq - t + 1) >> 1;             // blocks that see any
+  const int64_t a = p < all ? p : all, z0 = all > some ? all : some, z = p < z0 ? p : z0;
+  return a * nq + (z - a) * (nq - t) - (z * (z - 1) - a * (a - 1));
+}
+// A block of n steps is cut into ceil(n / iters) slices; the first slot of block p, counted like that, is at or before
+// floor(steps of the blocks before / iters) + p, which needs no sum over the blocks and leaves less than one slot unused each.
 struct BwdSlices {
   int32_t count;  // most slices of a key block
   int32_t iters;  // most steps (query head of the group, 64-row query tile) of a slice
+  int32_t slots;  // slots of 128 key rows: of each (sequence, kv head), packed: of each kv head, for all sequences
   size_t bytes;   // fp32 partial sums of dK, then of dV
 };
 inline BwdSlices bwd_slices(const fa_bwd_params* p) {
-  BwdSlices r = {1, 0x7fffffff, 0};
+  const BwdSlices whole = {1, 0x7fffffff, 0, 0};
   const int64_t group = p->heads_q / p->heads_k;
-  const int64_t units = (int64_t)p->batch * p->heads_k * ((p->seqlen_k + 127) / 128);
-  const int64_t longest = group * ((p->seqlen_q + 63) / 64);
-  if (units == 0 || longest == 0) return r;
+  const int64_t nk = ((int64_t)p->seqlen_k + 127) / 128, nq = ((int64_t)p->seqlen_q + 63) / 64;
+  const int64_t units = (int64_t)p->batch * p->heads_k * nk, longest = group * nq;
+  const bool causal = p->is_causal != FA_MASK_NONE;
+  if (units == 0 || longest == 0) return whole;
   // steps of all blocks; packed lengths are known on the device only, and sum(n^2) lies between total^2 / batch (equal
   // lengths) and total x longest: the geometric mean of the two, with a margin for being an estimate
-  double total = (double)units * (double)longest * (p->is_causal != FA_MASK_NONE ? 0.5 : 1.0), margin = 1.0;
+  double total = (double)units * (double)longest * (causal ? 0.5 : 1.0), margin = 1.0;
   if (p->cu_seqlens_q) {
     const double fill = (double)p->total_q / ((double)p->batch * p->seqlen_q);
     if (fill < 1.0) total *= fill * sqrt(fill);
     margin = 1.25;
   }
   const double spread = total / 256.0 * (p->head_dim <= 64 ? 1.2 : 1.75);
-  if ((double)longest <= margin * (spread + 10.0)) return r;
-  // about four slices per CU (of each kind), of 16 steps at least
-  int64_t want = (int64_t)(total / 1024.0);
+  if ((double)longest <= margin * (spread + 10.0)) return whole;
+  // about three slices per CU (of each kind), of 16 steps at least
+  int64_t want = (int64_t)(total / 832.0);
   if (want < 16) want = 16;
   int64_t n = (longest + want - 1) / want;
   if (n > FA_MAX_SPLITS) n = FA_MAX_SPLITS;
+  // steps and key blocks that share an array of slots: dense, those of a (sequence, kv head); packed, those of a kv head, as
+  // many as self-attention over total_q rows can have (sequences beyond that stay whole)
+  const int64_t rows_q = p->cu_seqlens_q ? p->total_q : (int64_t)p->batch * p->seqlen_q;
+  double steps, blocks;
+  if (p->cu_seqlens_q) {
+    steps = (double)group * ((double)p->total_q / 64 + p->batch) * (causal ? (double)nk / 2 + 1 : (double)nk);
+    blocks = (double)p->total_q / 128 + p->batch;
+  } else {
+    const int64_t off = p->is_causal == FA_MASK_CAUSAL_TOP_LEFT ? 0 : (int64_t)p->seqlen_k - p->seqlen_q;
+    steps = (double)group * (double)key_block_tiles_before(nk, nq, off, causal);
+    blocks = (double)nk;
+  }
+  const int64_t arrays = p->cu_seqlens_q ? p->heads_k : (int64_t)p->batch * p->heads_k;
   const int64_t slot = (int64_t)128 * padded_dim(p->head_dim) * 4 * 2;
-  while (n > 1 && units > (1LL << 30) / (slot * n)) --n;
-  if (n <= 1) return r;
-  r.count = (int32_t)n;
-  r.iters = (int32_t)((longest + n - 1) / n);
-  r.bytes = (size_t)(units * n * slot);
-  return r;
+  int64_t rows_k = (int64_t)p->batch * p->seqlen_k;
+  if (p->cu_seqlens_q && rows_k > rows_q) rows_k = rows_q;
+  const double tensors = 8.0 * p->head_dim * ((double)rows_q * p->heads_q + (double)rows_k * p->heads_k);
+  const double most = 1.25 * tensors < (double)(1LL << 30) ? 1.25 * tensors : (double)(1LL << 30);
+  for (; n > 1; --n) {
+    const int64_t iters = (longest + n - 1) / n;
+    const double slots = floor(steps / (double)iters) + ceil(blocks);
+    if (slots * (double)arrays * (double)slot > most || slots * (double)iters > (double)0x7fffffff) continue;
+    BwdSlices r;
+    r.count = (int32_t)n;
+    r.iters = (int32_t)iters;
+    r.slots = (int32_t)slots;
+    r.bytes = (size_t)r.slots * (size_t)arrays * (size_t)slot;
+    return r;
+  }
+  return whole;
 }
 inline size_t bwd_ws_bytes(const fa_bwd_params* p) { return 2 * bwd_ws_plane(p) + bwd_slices(p).bytes; }
 
