@@ -109,8 +109,8 @@ typedef struct fa_bwd_params {
 FA_API int fa_bwd_validate(const fa_bwd_params* p);
 
 /* Bytes of device scratch fa_bwd_launch needs (-rowsum(dO o O) and LSE log2(e), two fp32 per query row and head; and,
-   where the work of a key block is cut into slices, the slices' fp32 sums of dK and dV: at most 5/4 of the bytes that q,
-   out, dout, dq, k, v, dk and dv have together, and at most 1 GiB); 0 if invalid. */
+   where the work of a key block is cut into slices, the slices' fp32 sums of dK and dV: at most four times the bytes
+   that q, out, dout, dq, k, v, dk and dv have together, and at most 1 GiB); 0 if invalid. */
 FA_API size_t fa_bwd_workspace_bytes(const fa_bwd_params* p);
 
 /* Enqueue the backward pass on `stream`; `workspace` should hold fa_bwd_workspace_bytes(p) bytes, 16-byte aligned.  With

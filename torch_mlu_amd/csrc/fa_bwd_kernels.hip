@@ -101,6 +101,7 @@ struct BArgs {
   int64_t part_dv;            // floats from the partials of dK to those of dV
   int32_t n_slices, slice_iters;
   int32_t part_slots;         // slots of 128 key rows: of each (sequence, kv head); packed: of each kv head
+  uint64_t part_row, part_seq;  // packed: slots per row and per sequence before a sequence, times 2^32
 };
 
 // slices of a key block with `niter` steps: as even as possible, none longer than slice_iters
@@ -108,37 +109,26 @@ __device__ __forceinline__ int dkv_slices(const BArgs& a, int niter) {
   return min(a.n_slices, max(1, (niter + a.slice_iters - 1) / a.slice_iters));
 }
 
-// Slot of the first slice of key block `pslot` of sequence b (Lq rows, Lk keys), kv head hk, among the partial sums; -1: there
-// is no room for this sequence, its blocks stay whole (packed only, where the host knows the total length but not the
-// sequences').  Every lane of the wavefront calls it.  The dense products fit 31 bits (bwd_slices); a packed sequence whose
-// products do not is one there is no room for.
-__device__ __forceinline__ int dkv_first_slot(const BArgs& a, int b, int hk, int pslot, int Lq, int Lk) {
-  auto before = [&](int64_t p, int lq, int lk) -> int64_t {  // steps of the first p key blocks of a sequence
-    return fa::host::key_block_tiles_before(p, (lq + 63) / 64, a.causal_tl ? 0 : lk - lq, a.is_causal != 0) * a.group;
+// Slot of the first slice of key block `pslot` of sequence b (rows q0 ... q0 + Lq - 1, Lk keys), kv head hk, among the partial
+// sums; -1: there is no room for this sequence, its blocks stay whole.  Dense: every (sequence, kv head) has part_slots, enough
+// for all its blocks.  Packed, where the host does not know the lengths: a sequence has room in proportion to its rows, as much
+// as self-attention can need, which is found from its offset alone.
+__device__ __forceinline__ int dkv_first_slot(const BArgs& a, int b, int hk, int pslot, int q0, int Lq, int Lk) {
+  auto before = [&](int64_t p) -> int64_t {  // steps of the first p key blocks
+    return fa::host::key_block_tiles_before(p, (Lq + 63) / 64, a.causal_tl ? 0 : Lk - Lq, a.is_causal != 0) * a.group;
   };
   const unsigned iters = (unsigned)a.slice_iters;
-  const int mine = (int)((unsigned)before(pslot, Lq, Lk) / iters) + pslot;
+  const int mine = (int)((unsigned)before(pslot) / iters) + pslot;
   if (!a.cu_q) return (b * a.heads_k + hk) * a.part_slots + mine;
-  // slots of each sequence up to this one, a lane each; sums are cut off where they exceed what there is
-  const int lane = threadIdx.x & 63, cap = a.part_slots + 1;
-  int base = 0, own = 0;
-  for (int s0 = 0; s0 <= b; s0 += 64) {
-    const int s = s0 + lane;
-    int slots = 0;
-    if (s <= b) {
-      const int lq = max(a.cu_q[s + 1] - a.cu_q[s], 0), lk = max(a.cu_k[s + 1] - a.cu_k[s], 0);
-      const int nk = (lk + 127) / 128;
-      const int64_t steps = before(nk, lq, lk);
-      slots = steps > 0x7fffffff ? cap : (int)min((unsigned)steps / iters + (unsigned)nk, (unsigned)cap);
-    }
-    if (b - s0 < 64) own = __builtin_amdgcn_readlane(slots, __builtin_amdgcn_readfirstlane(b - s0));
-    if (s >= b) slots = 0;
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) slots += __shfl_xor(slots, o);
-    base = min(base + __builtin_amdgcn_readfirstlane(slots), cap);
-  }
-  if (base + own > a.part_slots) return -1;
-  return base * a.heads_k + hk * own + mine;
+  auto first = [&](int row, int seq) -> int {  // (never more than there are, whatever the offsets)
+    const uint64_t f = ((uint64_t)(unsigned)row * a.part_row + (uint64_t)(unsigned)seq * a.part_seq) >> 32;
+    return f < (uint64_t)a.part_slots ? (int)f : a.part_slots;
+  };
+  const int base = first(q0, b), room = first(q0 + Lq, b + 1) - base;
+  const int nk = (Lk + 127) / 128;
+  const int64_t steps = before(nk);
+  if (steps > 0x7fffffff || (int64_t)((unsigned)steps / iters) + nk > room) return -1;
+  return base * a.heads_k + hk * room + mine;
 }
 
 // One swizzle for tiles that are read both by rows (16 lanes = 16 consecutive rows, same logical chunk) and
@@ -721,11 +711,18 @@ __device__ __forceinline__ void dkv_block(const BArgs& a, unsigned char* smem, i
   const int jq_end = (Lq + BQ - 1) / BQ;
   const int nq = max(0, jq_end - jq_begin);
   // flattened (query head of the group, query tile); a slice takes steps it0 ... it1 - 1
-  const int niter = nq * a.group;
-  int it0 = 0, it1 = niter, ns = 1;
+  int it0 = 0, it1 = nq * a.group, slot = -1;
   if (a.n_slices > 1) {
-    ns = dkv_slices(a, niter);
+    int ns = dkv_slices(a, it1);
+    if (ns > 1) slot = dkv_first_slot(a, b, hk, pslot, q0, Lq, Lk);
+    if (slot < 0) ns = 1;
     if (slice >= ns) return;
+    if (ns > 1) {
+      slot += slice;
+      const int64_t n = it1;
+      it0 = (int)(n * slice / ns);
+      it1 = (int)(n * (slice + 1) / ns);
+    }
   }
 
   // ---- K and V fragments of my key row (B operands) ----
@@ -744,19 +741,6 @@ __device__ __forceinline__ void dkv_block(const BArgs& a, unsigned char* smem, i
       }
       kf[ks] = __builtin_bit_cast(s16x8, x);
       vf[ks] = __builtin_bit_cast(s16x8, y);
-    }
-  }
-
-  int slot = 0;
-  if (ns > 1) {  // (behind the loads above, which cover the look at the other sequences' lengths)
-    slot = dkv_first_slot(a, b, hk, pslot, Lq, Lk);
-    if (slot < 0) {
-      if (slice > 0) return;
-      ns = 1;
-    } else {
-      slot += slice;
-      it0 = (int)((int64_t)niter * slice / ns);
-      it1 = (int)((int64_t)niter * (slice + 1) / ns);
     }
   }
 
@@ -1002,11 +986,20 @@ __device__ __forceinline__ void dkv_block(const BArgs& a, unsigned char* smem, i
       {
         // Q (and dO) row fragments are fetched RS k-steps ahead of the MFMAs that consume them (a ring of RS slots)
         constexpr int RS = FA_RS(DO_K, DO_V) < KS ? FA_RS(DO_K, DO_V) : KS;
+        // k-step ks is 2 ks chunks of 16 bytes on, under the swizzle an exclusive or; with dropout at head_dim 128 seven
+        // addresses kept over the loop would spill, and reloading them waits for the next tile's DMA as well
+        LDS_AS const unsigned char* row0 = (LDS_AS const unsigned char*)qt + kaddr[0];
+        auto row_frag = [&](bool dout, int ks) -> s16x8 {
+          if constexpr (DROP && DP == 128)
+            return *(LDS_AS const s16x8*)((LDS_AS const unsigned char*)(uintptr_t)((unsigned)(uintptr_t)row0 ^ (32u * ks)) +
+                                          qbk * 32 * ROWB + (dout ? 2 * TILE : 0));
+          return *(const s16x8*)((dout ? dt : qt) + kaddr[ks] + qbk * 32 * ROWB);
+        };
         s16x8 qa[RS], da[RS];
 #pragma unroll
         for (int ks = 0; ks < RS; ++ks) {
-          qa[ks] = *(const s16x8*)(qt + kaddr[ks] + qbk * 32 * ROWB);
-          if constexpr (DO_K) da[ks] = *(const s16x8*)(dt + kaddr[ks] + qbk * 32 * ROWB);
+          qa[ks] = row_frag(false, ks);
+          if constexpr (DO_K) da[ks] = row_frag(true, ks);
         }
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -1014,8 +1007,8 @@ __device__ __forceinline__ void dkv_block(const BArgs& a, unsigned char* smem, i
           s = Mma<T>::m32(qa[ks % RS], kf[ks], s);
           if constexpr (DO_K) dp = Mma<T>::m32(da[ks % RS], vf[ks], dp);
           if (ks + RS < KS) {
-            qa[ks % RS] = *(const s16x8*)(qt + kaddr[ks + RS] + qbk * 32 * ROWB);
-            if constexpr (DO_K) da[ks % RS] = *(const s16x8*)(dt + kaddr[ks + RS] + qbk * 32 * ROWB);
+            qa[ks % RS] = row_frag(false, ks + RS);
+            if constexpr (DO_K) da[ks % RS] = row_frag(true, ks + RS);
           }
           __builtin_amdgcn_sched_barrier(0);
         }
@@ -1129,9 +1122,13 @@ __device__ __forceinline__ void dkv_block(const BArgs& a, unsigned char* smem, i
     }
   }
 
-  if (ns > 1) {
+  // this lane's numbers once more from its thread's: kept over the loop they cost registers that it does not have
+  int tid_e = threadIdx.x;
+  asm volatile("" : "+v"(tid_e));
+  const int lane_e = tid_e & 63, g_e = lane_e >> 5, c32_e = lane_e & 31;
+  if (slot >= 0) {
     // a slice's sums stay as the MFMAs left them: 16 bytes per lane, 1 KiB per store instruction
-    const int64_t at = ((int64_t)slot * 4 + wave) * (32 * DP) + lane * 4;
+    const int64_t at = ((int64_t)slot * 4 + wave) * (32 * DP) + lane_e * 4;
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
@@ -1152,7 +1149,7 @@ __device__ __forceinline__ void dkv_block(const BArgs& a, unsigned char* smem, i
     constexpr int OSTR = ROWB + 16;
     unsigned char* stage = smem + wave * (32 * OSTR);
     constexpr int RPS = 64 / CPR;  // rows per store instruction
-    const int sr = lane / CPR, sch = lane % CPR;
+    const int sr = lane_e / CPR, sch = lane_e % CPR;
     const int rows_left = Lk - (n0 + 32 * wave);
     const float sc = a.scale;
     auto flush = [&](unsigned char* base, int64_t row_stride) __attribute__((always_inline)) {
@@ -1171,7 +1168,7 @@ __device__ __forceinline__ void dkv_block(const BArgs& a, unsigned char* smem, i
           u32x2 w;
           w[0] = Mma<T>::pack2(dk[mb][4 * v4 + 0] * sc, dk[mb][4 * v4 + 1] * sc);
           w[1] = Mma<T>::pack2(dk[mb][4 * v4 + 2] * sc, dk[mb][4 * v4 + 3] * sc);
-          *(u32x2*)(stage + c32 * OSTR + (32 * mb + 8 * v4 + 4 * g) * 2) = w;
+          *(u32x2*)(stage + c32_e * OSTR + (32 * mb + 8 * v4 + 4 * g_e) * 2) = w;
         }
       flush(a.dk + dkb + (int64_t)(k0 + n0 + 32 * wave) * a.dk_ss + (int64_t)hk * a.dk_sh, a.dk_ss);
     }
@@ -1183,7 +1180,7 @@ __device__ __forceinline__ void dkv_block(const BArgs& a, unsigned char* smem, i
           u32x2 w;
           w[0] = Mma<T>::pack2(dv[mb][4 * v4 + 0], dv[mb][4 * v4 + 1]);
           w[1] = Mma<T>::pack2(dv[mb][4 * v4 + 2], dv[mb][4 * v4 + 3]);
-          *(u32x2*)(stage + c32 * OSTR + (32 * mb + 8 * v4 + 4 * g) * 2) = w;
+          *(u32x2*)(stage + c32_e * OSTR + (32 * mb + 8 * v4 + 4 * g_e) * 2) = w;
         }
       flush(a.dv + dvb + (int64_t)(k0 + n0 + 32 * wave) * a.dv_ss + (int64_t)hk * a.dv_sh, a.dv_ss);
     }
@@ -1232,9 +1229,10 @@ __global__ void __launch_bounds__(256) fa_bwd_dkv_merge_kernel(const BArgs a) {
   const int bhk = unit % nbh, pslot = unit / nbh;
   const int hk = bhk % a.heads_k, b = bhk / a.heads_k;
   const bool is_dv = blockIdx.y != 0;
-  int k0 = 0, Lq = a.seqlen_q, Lk = a.seqlen_k;
+  int q0 = 0, k0 = 0, Lq = a.seqlen_q, Lk = a.seqlen_k;
   if (a.cu_q) {
-    Lq = a.cu_q[b + 1] - a.cu_q[b];
+    q0 = a.cu_q[b];
+    Lq = a.cu_q[b + 1] - q0;
     k0 = a.cu_k[b];
     Lk = a.cu_k[b + 1] - k0;
   }
@@ -1245,7 +1243,7 @@ __global__ void __launch_bounds__(256) fa_bwd_dkv_merge_kernel(const BArgs a) {
   const int jq_begin = a.is_causal ? max(0, n0 - off) / BQ : 0;
   const int ns = dkv_slices(a, max(0, (Lq + BQ - 1) / BQ - jq_begin) * a.group);
   if (ns == 1) return;  // written by the dK/dV kernel
-  const int slot = dkv_first_slot(a, b, hk, pslot, Lq, Lk);
+  const int slot = dkv_first_slot(a, b, hk, pslot, q0, Lq, Lk);
   if (slot < 0) return;
   const float* src = a.part + (is_dv ? a.part_dv : 0) + ((int64_t)slot * 4 + part) * (32 * DP) + tid * 4;
   f32x4 sum[MB];
@@ -1365,6 +1363,7 @@ int fa_bwd_launch(const fa_bwd_params* p, void* workspace, size_t workspace_byte
   host::BwdSlices sl = host::bwd_slices(p);
   if (workspace_bytes < need) sl.count = 1;  // no room for partial sums: whole key blocks
   a.n_slices = sl.count; a.slice_iters = sl.iters; a.part_slots = sl.slots;
+  a.part_row = sl.per_row; a.part_seq = sl.per_seq;
   a.part = (float*)((unsigned char*)workspace + 2 * bwd_ws_plane(p));
   a.part_dv = (int64_t)(sl.bytes / 8);
   a.cu_q = p->cu_seqlens_q; a.cu_k = p->cu_seqlens_k;

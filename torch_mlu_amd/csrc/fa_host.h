@@ -287,8 +287,9 @@ inline size_t bwd_ws_plane(const fa_bwd_params* p) {
 // 2048 rows 225 -> 165; 8 packed sequences of 187 ... 1500 rows, 16 / 4, 250 -> 232.  On the other side of the line:
 // 16 / 16, 2048 rows 113 -> 133; 8 / 8, 4096 rows 209 -> 222; batch 2, 16 / 8, head_dim 256, 2000 rows 331 -> 423.
 //
-// The partial sums take at most 5/4 of the memory of the call's own tensors (q, out, dout, dq and k, v, dk, dv): slices get
-// longer until they do, or the blocks stay whole.
+// The partial sums take at most four times the memory of the call's own tensors (q, out, dout, dq and k, v, dk, dv), which
+// one kv head for many query heads comes near (8 / 1 heads, 4096 rows: 128 MiB beside 34; twice would cost it 6 %): slices
+// get longer until they do, or the blocks stay whole.
 //
 // Pairs of (128-key block, 64-row query tile that sees some of its keys) in the first p key blocks: off = Lk - Lq, or 0 for
 // the top-left mask.  Block i sees the tiles from max(0, 128 i - off) / 64 = max(0, 2 i + t) on.  (constexpr: the kernels
@@ -308,9 +309,10 @@ struct BwdSlices {
   int32_t iters;  // most steps (query head of the group, 64-row query tile) of a slice
   int32_t slots;  // slots of 128 key rows: of each (sequence, kv head), packed: of each kv head, for all sequences
   size_t bytes;   // fp32 partial sums of dK, then of dV
+  uint64_t per_row, per_seq;  // packed: slots that a row and a sequence add to the first slot of the next one, times 2^32
 };
 inline BwdSlices bwd_slices(const fa_bwd_params* p) {
-  const BwdSlices whole = {1, 0x7fffffff, 0, 0};
+  const BwdSlices whole = {1, 0x7fffffff, 0, 0, 0, 0};
   const int64_t group = p->heads_q / p->heads_k;
   const int64_t nk = ((int64_t)p->seqlen_k + 127) / 128, nq = ((int64_t)p->seqlen_q + 63) / 64;
   const int64_t units = (int64_t)p->batch * p->heads_k * nk, longest = group * nq;
@@ -326,38 +328,40 @@ inline BwdSlices bwd_slices(const fa_bwd_params* p) {
   }
   const double spread = total / 256.0 * (p->head_dim <= 64 ? 1.2 : 1.75);
   if ((double)longest <= margin * (spread + 10.0)) return whole;
-  // about three slices per CU (of each kind), of 16 steps at least
-  int64_t want = (int64_t)(total / 832.0);
+  // slices of 16 steps at least; about three per CU of each kind where dK and dV share a launch, else four (28 query / 4 kv
+  // heads, 4096 rows, dropout: 1067 us with four, 1126 with three; head_dim 256, 16 / 2, 4096 rows, causal: 775 and 721)
+  const bool alone = p->head_dim <= 64 || p->dropout_p > 0.f || p->bias;
+  int64_t want = (int64_t)(total / (alone ? 1024.0 : 832.0));
   if (want < 16) want = 16;
   int64_t n = (longest + want - 1) / want;
   if (n > FA_MAX_SPLITS) n = FA_MAX_SPLITS;
-  // steps and key blocks that share an array of slots: dense, those of a (sequence, kv head); packed, those of a kv head, as
-  // many as self-attention over total_q rows can have (sequences beyond that stay whole)
+  // steps and key blocks that share an array of slots: dense, those of a (sequence, kv head); packed, those of a kv head.
+  // There a sequence of L rows gets room for as many as self-attention can have, at most L / 64 + 1 query tiles times (of a
+  // causal mask half) the key blocks of the longest, and L / 128 + 1 blocks; one with more keys than that stays whole
   const int64_t rows_q = p->cu_seqlens_q ? p->total_q : (int64_t)p->batch * p->seqlen_q;
-  double steps, blocks;
-  if (p->cu_seqlens_q) {
-    steps = (double)group * ((double)p->total_q / 64 + p->batch) * (causal ? (double)nk / 2 + 1 : (double)nk);
-    blocks = (double)p->total_q / 128 + p->batch;
-  } else {
-    const int64_t off = p->is_causal == FA_MASK_CAUSAL_TOP_LEFT ? 0 : (int64_t)p->seqlen_k - p->seqlen_q;
-    steps = (double)group * (double)key_block_tiles_before(nk, nq, off, causal);
-    blocks = (double)nk;
-  }
+  const double wide = causal ? 0.5 * (double)nk + 1.0 : (double)nk;
+  const int64_t off = p->is_causal == FA_MASK_CAUSAL_TOP_LEFT ? 0 : (int64_t)p->seqlen_k - p->seqlen_q;
+  const double steps = (double)group * (double)key_block_tiles_before(nk, nq, off, causal);
   const int64_t arrays = p->cu_seqlens_q ? p->heads_k : (int64_t)p->batch * p->heads_k;
   const int64_t slot = (int64_t)128 * padded_dim(p->head_dim) * 4 * 2;
   int64_t rows_k = (int64_t)p->batch * p->seqlen_k;
   if (p->cu_seqlens_q && rows_k > rows_q) rows_k = rows_q;
   const double tensors = 8.0 * p->head_dim * ((double)rows_q * p->heads_q + (double)rows_k * p->heads_k);
-  const double most = 1.25 * tensors < (double)(1LL << 30) ? 1.25 * tensors : (double)(1LL << 30);
+  const double most = 4.0 * tensors < (double)(1LL << 30) ? 4.0 * tensors : (double)(1LL << 30);
   for (; n > 1; --n) {
     const int64_t iters = (longest + n - 1) / n;
-    const double slots = floor(steps / (double)iters) + ceil(blocks);
+    const double tile = (double)group * wide / (double)iters;  // packed: slots per query tile
+    const double per_row = tile / 64 + 1.0 / 128, per_seq = tile + 1.0;
+    const double slots = p->cu_seqlens_q ? ceil((double)p->total_q * per_row + (double)p->batch * per_seq)
+                                         : floor(steps / (double)iters) + (double)nk;
     if (slots * (double)arrays * (double)slot > most || slots * (double)iters > (double)0x7fffffff) continue;
     BwdSlices r;
     r.count = (int32_t)n;
     r.iters = (int32_t)iters;
     r.slots = (int32_t)slots;
     r.bytes = (size_t)r.slots * (size_t)arrays * (size_t)slot;
+    r.per_row = (uint64_t)ceil(per_row * 4294967296.0);
+    r.per_seq = (uint64_t)ceil(per_seq * 4294967296.0);
     return r;
   }
   return whole;
