@@ -1,10 +1,13 @@
 """Work distribution of the forward kernels: every (sequence, head, row) is computed once, whatever order the blocks run
 in and however many slices are merged.  Results against float32 math on the device (bars: tests/_util.py)."""
+import ctypes
 import math
 
+import numpy as np
 import pytest
 import torch
 
+import oracle
 from tests._util import LSE_TOL, OUT_TOL
 from torch_mlu_amd import capi
 
@@ -145,8 +148,9 @@ def test_ragged_paged_units_around_one_per_cu(D, B, per, ns):
     assert (lse[:, :, 0] - want_l).abs().max().item() <= LSE_TOL
 
 
-def _grad_reference(q, k, v, do, causal, bias=None):
-    """Gradients of one dense call in float64 on the CPU."""
+def _grad_reference(q, k, v, do, causal, bias=None, keep=None, keep_p=1.0):
+    """Gradients of one dense call in float64 on the CPU.  `causal`: False, True or a mask mode; `keep`: the elements that
+    dropout kept, `keep_p` of them."""
     q, k, v, do = (t.double().cpu() for t in (q, k, v, do))
     g, D, Sq, Sk = q.shape[1] // k.shape[1], q.shape[3], q.shape[2], k.shape[2]
     kr, vr = k.repeat_interleave(g, 1), v.repeat_interleave(g, 1)
@@ -154,13 +158,15 @@ def _grad_reference(q, k, v, do, causal, bias=None):
     if bias is not None:
         s = s + bias.double().cpu()
     if causal:
-        s.masked_fill_(~(torch.arange(Sk)[None, :] <= torch.arange(Sq)[:, None] + Sk - Sq), float("-inf"))
+        off = 0 if int(causal) == capi.FA_MASK_CAUSAL_TOP_LEFT else Sk - Sq
+        s.masked_fill_(~(torch.arange(Sk)[None, :] <= torch.arange(Sq)[:, None] + off), float("-inf"))
     p = torch.nan_to_num(torch.softmax(s, -1))
-    dp = do @ vr.transpose(2, 3)
+    m = 1.0 if keep is None else keep.double().cpu() / keep_p
+    dp = do @ vr.transpose(2, 3) * m
     ds = p * (dp - (p * dp).sum(-1, keepdim=True)) / math.sqrt(D)
     B, Hk = k.shape[:2]
     fold = lambda t: t.reshape(B, Hk, g, Sk, D).sum(2)
-    return ds @ kr, fold(ds.transpose(2, 3) @ q), fold(p.transpose(2, 3) @ do)
+    return ds @ kr, fold(ds.transpose(2, 3) @ q), fold((p * m).transpose(2, 3) @ do)
 
 
 def _check_grads(got, want, dtype):
@@ -194,6 +200,67 @@ def test_sliced_key_blocks_with_a_bias(D):
     bias = _randn((1, 1, 260, 200), 34, BF)
     out, lse = capi.fa_forward_dense(q, k, v, bias=bias)
     _check_grads(capi.fa_backward_dense(do, q, k, v, out, lse, bias=bias)[:3], _grad_reference(q, k, v, do, False, bias), BF)
+
+
+@pytest.fixture
+def sliced(monkeypatch):
+    """Every backward call of the test cuts key blocks: it asks for more than the two planes of its rows."""
+    launch = capi._launch_bwd
+
+    def checked(p, device):
+        rows = p.total_q if p.cu_seqlens_q else p.batch * p.seqlen_q
+        assert capi.lib().fa_bwd_workspace_bytes(ctypes.byref(p)) > 2 * (rows * p.heads_q * 4 + 15)
+        launch(p, device)
+
+    monkeypatch.setattr(capi, "_launch_bwd", checked)
+
+
+@pytest.mark.parametrize("D", [64, 72, 128, 256])
+@pytest.mark.parametrize("B,Hq,Hk,Sq,Sk", [
+    (1, 14, 2, 130, 130),
+    (1, 14, 2, 500, 300),    # the last rows see every key, as many as there are
+    (1, 14, 2, 300, 700),    # the last keys are seen by no row
+])
+def test_sliced_key_blocks_top_left(sliced, D, B, Hq, Hk, Sq, Sk):
+    mode = capi.FA_MASK_CAUSAL_TOP_LEFT
+    q, k, v, do = (_randn(s, 80 + i, BF) for i, s in enumerate([(B, Hq, Sq, D), (B, Hk, Sk, D), (B, Hk, Sk, D), (B, Hq, Sq, D)]))
+    out, lse = capi.fa_forward_dense(q, k, v, is_causal=mode)
+    _check_grads(capi.fa_backward_dense(do, q, k, v, out, lse, is_causal=mode), _grad_reference(q, k, v, do, mode), BF)
+
+
+@pytest.mark.parametrize("with_bias", [False, True])
+@pytest.mark.parametrize("D", [64, 128, 256])
+@pytest.mark.parametrize("B,Hq,Hk,Sq,Sk,causal", [
+    (1, 14, 2, 260, 260, True),
+    (2, 21, 3, 400, 132, False),
+    (1, 16, 1, 200, 388, capi.FA_MASK_CAUSAL_TOP_LEFT),
+])
+def test_sliced_key_blocks_with_dropout(sliced, D, B, Hq, Hk, Sq, Sk, causal, with_bias):
+    q, k, v, do = (_randn(s, 90 + i, HF) for i, s in enumerate([(B, Hq, Sq, D), (B, Hk, Sk, D), (B, Hk, Sk, D), (B, Hq, Sq, D)]))
+    bias = _randn((B, 1, Sq, Sk), 94, HF) if with_bias else None
+    rng, mask = torch.zeros(2, dtype=torch.int64, device=DEV), torch.zeros((B, Hq, Sq, Sk), dtype=HF, device=DEV)
+    out, lse = capi.fa_forward_dense(q, k, v, is_causal=causal, bias=bias, dropout_p=0.2, philox_seed=11, philox_offset=4,
+                                     rng_out=rng, dropout_mask=mask)
+    got = capi.fa_backward_dense(do, q, k, v, out, lse, is_causal=causal, bias=bias, dropout_p=0.2, rng=rng)
+    keep_p = (math.floor(np.float32(1.0 - np.float32(0.2)) * np.float32(255.0)) + 1) / 256
+    _check_grads(got[:3], _grad_reference(q, k, v, do, causal, bias, mask > 0, keep_p), HF)
+
+
+def test_sliced_key_blocks_packed_with_dropout(sliced):
+    # (no sequence of one row: its dK is exactly 0, and what a kernel gives instead is the rounding of O in delta, up to
+    # heads x scale x |q| x 2^-11 x sum |dO| |O| = 7 x 0.09 x 2 x 2^-11 x 30 = 0.02 here, which the bar below does not count)
+    lens, Hq, Hk, D, drop = [300, 33, 520, 64], 14, 2, 128, 0.3
+    cu = np.concatenate([[0], np.cumsum(lens)]).tolist()
+    q, k, v, do = (_randn(s, 100 + i, HF) for i, s in enumerate([(cu[-1], Hq, D), (cu[-1], Hk, D), (cu[-1], Hk, D), (cu[-1], Hq, D)]))
+    c, rng = torch.tensor(cu, dtype=torch.int32, device=DEV), torch.zeros(2, dtype=torch.int64, device=DEV)
+    out, lse = capi.fa_forward_packed(q, k, v, c, c, max(lens), max(lens), is_causal=True, dropout_p=drop, philox_seed=5,
+                                      philox_offset=12, rng_out=rng)
+    got = capi.fa_backward_packed(do, q, k, v, out, lse, c, c, max(lens), max(lens), is_causal=True, dropout_p=drop, rng=rng)
+    row = lambda t, i: t[cu[i]:cu[i + 1]].transpose(0, 1)[None]
+    for i, n in enumerate(lens):
+        keep = torch.from_numpy(np.stack([oracle.dropout_keep_mask(5, 12, i * Hq + h, n, n, drop) for h in range(Hq)]))[None]
+        want = _grad_reference(*(row(t, i) for t in (q, k, v, do)), True, None, keep, 1.0 - oracle.dropout_effective_p(drop))
+        _check_grads([row(t, i) for t in got], want, HF)
 
 
 @pytest.mark.parametrize("Hq,Hk,D", [(14, 2, 64), (14, 2, 128), (8, 1, 96)])
